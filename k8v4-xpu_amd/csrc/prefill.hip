@@ -21,7 +21,10 @@
 //    the score tile is already the B operand of the PV product.
 //  * K codes become fp16 integers (byte permute into the mantissa of 1024.0,
 //    then subtract 1152) times the token's K scale and the exp2-domain
-//    softmax factor (one fp16 rounding, as a bf16/fp16 dequant has).
+//    softmax factor, rounded to fp16: in tile images the fp32 product once
+//    (error of a 4,224-token chunk over 131,072 against float64: 8.1e-4
+//    relative, 1.8e-3 with the factor rounded to fp16 first), in place as a
+//    packed fp16 multiply by the rounded factor.
 //  * Online softmax in the exp2 domain with a lazy rescale (the running max
 //    only moves when a row's max grows by more than 2^2).
 //  * Head dim 128 (run_segment_pp): eight waves in two groups that alternate
@@ -30,8 +33,10 @@
 //    ((nibble - v_zero) * v_scale / 16, one fp16 rounding) and the softmax
 //    row sums come from the PV product itself (an extra MFMA against a ones
 //    row), so the softmax is max, exp2 and one conversion per score.
-//  * Head dim 256 (run_segment): four waves (the register file holds the wider
-//    accumulators) that convert each page together, then multiply.  V
+//  * Head dim 256 over tile images (run_segment_pair): two waves share 64 rows
+//    and interleave the vector work with the products in their own instruction
+//    streams.  In place (run_segment): four waves of 32 rows that convert each
+//    page together, then multiply.  V
 //    nibbles become exact fp16 subnormals (n * 2^-24 for even dims,
 //    16 n * 2^-24 for odd dims) in a transposed tile, the V scale multiplies
 //    P and the zero point is subtracted once per row at the end:
@@ -39,6 +44,7 @@
 #include "k8v4_common.h"
 
 #include <algorithm>
+#include <utility>
 #include <vector>
 
 namespace k8v4 {
@@ -82,7 +88,7 @@ struct PrefillArgs {
   int xcd_perm;  // map ids so the work-groups of one XCD take adjacent work (grid % 8 == 0)
   float *ws;     // partial states: [grid][2][rows][D + 2] floats
   int head0;     // KV head of step 0 (a launch covers heads head0 .. head0 + total / tper - 1)
-  const char *tiles;  // dequantized tiles of head head0, [page][PP::BUF] (D = 128) or [page][Tile<256>::TBUF] bytes (null: convert in-kernel)
+  const char *tiles;  // dequantized tiles of head head0, [page][PP::BUF] (D = 128) or [page][PW256::IMG] bytes (null: convert in-kernel)
   void *out;
   int out_dtype;
   int64_t out_tok_stride;  // elements
@@ -121,11 +127,6 @@ struct Tile {
   static constexpr int VDMA = D / 32;                 // 1 KB V pieces per page
   static constexpr int KCHUNKS = 4 * D;               // 16-byte K code chunks per page
   static constexpr int VITEMS = 2 * D;                // (part, half, key pair) V items per page
-  // Tile images dequantized beforehand (D = 256): one per page in the
-  // workspace, BUF rounded up to whole 1 KB pieces, each piece one DMA of a
-  // wave; the ring then holds two such images.
-  static constexpr int TBUF = (BUF + 1023) / 1024 * 1024;
-  static constexpr int TPIECES = TBUF / 1024;
 };
 
 typedef const __attribute__((address_space(4))) int32_t *const_i32_ptr;
@@ -197,7 +198,23 @@ __device__ __forceinline__ void k_codes_to_f16(uint32_t w, v2h &lo, v2h &hi) {
   hi = __builtin_bit_cast(v2h, b) - bias;
 }
 
-template <int D>
+// Codes times a factor, rounded to fp16 once.  IMG (tile images, converted once
+// per call): the factor stays fp32.  In place, where every row block converts
+// again: a packed multiply by the factor in fp16, a second rounding.
+template <bool IMG>
+__device__ __forceinline__ void scale_codes(v2h (&h)[8], float f) {
+  if constexpr (IMG) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      h[e] = (v2h){static_cast<_Float16>(static_cast<float>(h[e][0]) * f), static_cast<_Float16>(static_cast<float>(h[e][1]) * f)};
+  } else {
+    const v2h f2 = {static_cast<_Float16>(f), static_cast<_Float16>(f)};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) h[e] *= f2;
+  }
+}
+
+template <int D, bool IMG = false>
 __device__ __forceinline__ void convert_page(const PrefillArgs &a, int p, const char *stage, char *buf, int tid) {
   using T = Tile<D>;
 #pragma unroll
@@ -210,14 +227,12 @@ __device__ __forceinline__ void convert_page(const PrefillArgs &a, int p, const 
     // key past the sequence gets 0: its unwritten plane may hold anything).
     const float ks = reinterpret_cast<const float *>(buf + T::S_OFF)[key];
     const float kc = p * 64 + key < a.seq_len ? ks * a.c : 0.f;
-    const v2h kc2 = {static_cast<_Float16>(kc), static_cast<_Float16>(kc)};
     v2h h[8];
     k_codes_to_f16(w.x, h[0], h[1]);
     k_codes_to_f16(w.y, h[2], h[3]);
     k_codes_to_f16(w.z, h[4], h[5]);
     k_codes_to_f16(w.w, h[6], h[7]);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) h[e] *= kc2;
+    scale_codes<IMG>(h, kc);
     char *row = buf + key * T::KROW;
     const uint4 c0 = make_uint4(__builtin_bit_cast(uint32_t, h[0]), __builtin_bit_cast(uint32_t, h[1]),
                                 __builtin_bit_cast(uint32_t, h[2]), __builtin_bit_cast(uint32_t, h[3]));
@@ -323,16 +338,10 @@ __device__ __forceinline__ int range_owner(const PrefillArgs &a, int s) {
 
 // One segment: pages [p_lo, p_hi) of row block rb of KV head h.  `part` is
 // null when the segment is the whole block (the output is written directly).
-//
-// PRE (D = 256): the pages' tile images were dequantized beforehand
-// (prefill_convert256_kernel writes each page's image to a.tiles once for
-// all row blocks of the head): the ring's two buffers (TBUF apart) receive
-// them by DMA, and the waves only multiply.
-template <int D, bool PRE = false>
+template <int D>
 __device__ __forceinline__ void run_segment(const PrefillArgs &a, char *smem, int h, int rb, int p_lo, int p_hi,
                                             float *part, int tid, int wave, int lane) {
   using T = Tile<D>;
-  constexpr int RB = PRE ? T::TBUF : T::BUF;  // ring buffer stride
   lds_t *stage_lds = (lds_t *)(smem + 2 * T::BUF);
   const char *stage = smem + 2 * T::BUF;
   const int nrows = a.q_len * 6;
@@ -387,37 +396,17 @@ __device__ __forceinline__ void run_segment(const PrefillArgs &a, char *smem, in
   const int k_base = r32 * T::KROW + 16 * hh;
   const int v_base = T::V_OFF + r32 * T::VROW + 16 * hh;
 
-  // PRE: wave w moves pieces w, w + NW, ... of a page's image.
-  auto tile_dma = [&](int p, int bi) {
-    const char *src = a.tiles + static_cast<int64_t>(p) * T::TBUF + 16 * lane;
-#pragma unroll
-    for (int j = 0; j < (T::TPIECES + T::NW - 1) / T::NW; ++j) {
-      const int k = T::NW * j + wave;
-      if (k < T::TPIECES) dma16(src + 1024 * k, (lds_t *)(smem + bi * RB + 1024 * k));
-    }
-  };
-  if constexpr (PRE) {
-    tile_dma(p_lo, 0);
-    wait_dma();
-    __syncthreads();
-  } else {
-    stage_page<D>(a, p_lo, h, wave, lane, stage_lds, (lds_t *)(smem + T::S_OFF));
-    wait_dma();
-    __syncthreads();
-    convert_page<D>(a, p_lo, stage, smem, tid);
-    __syncthreads();
-  }
+  stage_page<D>(a, p_lo, h, wave, lane, stage_lds, (lds_t *)(smem + T::S_OFF));
+  wait_dma();
+  __syncthreads();
+  convert_page<D>(a, p_lo, stage, smem, tid);
+  __syncthreads();
 
   for (int p = p_lo; p < p_hi; ++p) {
     const int bi = (p - p_lo) & 1;
-    const char *buf = smem + bi * RB;
+    const char *buf = smem + bi * T::BUF;
     const bool more = p + 1 < p_hi;
-    if (more) {
-      if constexpr (PRE)
-        tile_dma(p + 1, bi ^ 1);
-      else
-        stage_page<D>(a, p + 1, h, wave, lane, stage_lds, (lds_t *)(smem + (bi ^ 1) * T::BUF + T::S_OFF));
-    }
+    if (more) stage_page<D>(a, p + 1, h, wave, lane, stage_lds, (lds_t *)(smem + (bi ^ 1) * T::BUF + T::S_OFF));
 
     // ---- S^T = K Q^T - m for the 64 keys of page p: lane (r, hh) reg 4j+i
     // of tile mt holds key 32*mt + 8*j + 4*hh + i of row r.  The accumulators
@@ -518,10 +507,8 @@ __device__ __forceinline__ void run_segment(const PrefillArgs &a, char *smem, in
 
     if (more) {
       wait_dma();
-      if constexpr (!PRE) {
-        __syncthreads();
-        convert_page<D>(a, p + 1, stage, smem + (bi ^ 1) * T::BUF, tid);
-      }
+      __syncthreads();
+      convert_page<D>(a, p + 1, stage, smem + (bi ^ 1) * T::BUF, tid);
     }
     __syncthreads();
   }
@@ -727,14 +714,12 @@ __device__ __forceinline__ void tile_store(char *dst, T v) {
 template <bool NT = false>
 __device__ __forceinline__ void pp_emit_k(const PrefillArgs &a, int p, const PPKIn &in, char *buf, int kc_dst, int key) {
   const float kc = p * 64 + key < a.seq_len ? in.ks * a.c : 0.f;
-  const v2h kc2 = {static_cast<_Float16>(kc), static_cast<_Float16>(kc)};
   v2h h[8];
   k_codes_to_f16(in.k.x, h[0], h[1]);
   k_codes_to_f16(in.k.y, h[2], h[3]);
   k_codes_to_f16(in.k.z, h[4], h[5]);
   k_codes_to_f16(in.k.w, h[6], h[7]);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) h[e] *= kc2;
+  scale_codes<NT>(h, kc);
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   char *row = buf + kc_dst;
   tile_store<NT>(row, (u32x4){__builtin_bit_cast(uint32_t, h[0]), __builtin_bit_cast(uint32_t, h[1]),
@@ -1140,12 +1125,596 @@ __device__ __forceinline__ void run_segment_pp(const PrefillArgs &a, char *smem,
     }
 }
 
+// ---- order of the page steps over tile images
+// All work-groups of an XCD read their tiles through one 4 MB L2, and the
+// tiles of a long context are many times that.  Each work-group therefore
+// visits its pages in an order that depends on its step count only, so that
+// at any time the work-groups stand at a few common pages: with T steps per
+// work-group, a segment inside one block starts at the page that is a multiple
+// of T and wraps at its end (at step t it is at a page congruent to t); of a
+// work-group with the tail of one block and the head of the next, the head
+// comes first (page t) and the tail after it (page n - T + t, the same for
+// every such work-group of equal n).  The softmax does not depend on the order.
+struct PageOrder {
+  int p_lo, p_hi, start;  // pages start .. p_hi - 1, then p_lo .. start - 1
+  __device__ __forceinline__ int page(int i) const {
+    const int p = start + i;
+    return p < p_hi ? p : p - (p_hi - p_lo);
+  }
+};
+struct TileSegment {
+  int hl, rb, p_lo, p_hi, slot;
+  bool whole;
+  PageOrder order;
+};
+
+// The last segment of the steps [s0, e) of a work-group that owns [s0, s1).
+__device__ __forceinline__ TileSegment last_segment(const PrefillArgs &a, int s0, int s1, int e, int lane) {
+  TileSegment g;
+  g.hl = (e - 1) / a.tper;
+  int before;
+  locate_block(a, e - 1 - g.hl * a.tper, lane, g.rb, before);
+  const int base = g.hl * a.tper + before;
+  const int n = block_pages(a, g.rb);
+  g.p_lo = max(0, s0 - base);
+  g.p_hi = e - base;
+  g.slot = s0 >= base ? 0 : 1;
+  g.whole = g.p_lo == 0 && g.p_hi == n;
+  int start = g.p_lo;
+  if (g.whole) {
+    start = (s1 - e) % n;
+  } else if (s0 >= base && e == s1) {
+    const int T = a.total / a.grid + 1;
+    start = (g.p_lo + T - 1) / T * T;
+    if (start >= g.p_hi) start = g.p_lo;
+  }
+  g.order = PageOrder{g.p_lo, g.p_hi, start};
+  return g;
+}
+
+// ---- products of the tile-image paths, with the register files fixed: scores (and
+// the vector work on them) in VGPRs, O, the query and the operands read from
+// LDS in accumulation VGPRs; left to itself the compiler puts every product in
+// one file and copies or spills.  It does not see these as MFMAs: a result may
+// be read by another instruction kind only after mfma_settle() or four further
+// products.
+__device__ __forceinline__ void mfma_score0(v16f &d, v8h a, v8h b, const v16f &c) {
+  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "a"(b), "v"(c));
+}
+__device__ __forceinline__ void mfma_score(v16f &d, v8h a, v8h b) {
+  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "a"(b));
+}
+__device__ __forceinline__ void mfma_score0_v(v16f &d, v8h a, v8h b, const v16f &c) {
+  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "v"(b), "v"(c));
+}
+__device__ __forceinline__ void mfma_score_v(v16f &d, v8h a, v8h b) {
+  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma_out(v16f &d, v8h a, v8h b) {
+  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(d) : "a"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma_settle() {
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// o[e] *= f without the accumulator leaving its registers.
+__device__ __forceinline__ void acc_scale(v16f &o, int e, float f) {
+  float x = o[e], t;
+  asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\tv_accvgpr_write_b32 %0, %1"
+               : "+a"(x), "=&v"(t)
+               : "v"(f));
+  o[e] = x;
+}
+
+// DMAs of the wide paths: one or two consecutive 1 KB pieces (the immediate
+// offset moves both the source and the LDS address).  The base is copied by
+// the scalar unit first: the load may not read an SGPR within five states of a
+// vector write to it (a v_readlane, if the compiler spilled the base), and the
+// copy also is the state the load needs after the write of M0.
+__device__ __forceinline__ void dma_piece(const void *sbase, uint32_t voff, const lds_t *dst) {
+  uint64_t base;
+  asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0"
+               : "=&s"(base)
+               : "v"(voff), "s"(sbase), "s"(lds_addr(dst))
+               : "memory", "m0");
+}
+__device__ __forceinline__ void dma_piece_pair(const void *sbase, uint32_t voff, const lds_t *dst) {
+  uint64_t base;
+  asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0\n\t"
+               "global_load_lds_dwordx4 %1, %0 offset:1024"
+               : "=&s"(base)
+               : "v"(voff), "s"(sbase), "s"(lds_addr(dst))
+               : "memory", "m0");
+}
+
+// f(0), ..., f(N - 1) with constant indices (a body this long is past the
+// compiler's limit for unrolling a loop).
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// ---- D = 256 over tile images: pairs of waves share 64 rows ----
+// What bounds it: a wave that owns 32 rows reads one operand from LDS per MFMA
+// (64 KB per wave and page: at 128 B per clock the four waves of a work-group
+// need as many LDS clocks as matrix clocks), and with one wave per SIMD its
+// softmax, waits and barriers add to the products instead of running beside
+// them.  Here every operand read feeds two MFMAs, and the vector work of one
+// page is interleaved with the products of its neighbours in the wave's own
+// instruction stream.  A 64-row wave's query and output do not fit one wave's
+// registers at this head dim, so two waves share the rows: each computes the
+// scores of 32 of a page's 64 keys (all 256 dims) and the output of 128 of the
+// 256 dims (all 64 keys), and they exchange through LDS the fp16
+// probabilities of their keys and their row maxima.
+// Measured, 4,224 query tokens over 63,724 keys, 2 KV heads: 4,897 -> 2,880
+// us (648 -> 1,110 TFLOP/s); a large fp16 matrix product reaches 1,318
+// TFLOP/s on this card, at the same power limit.
+//
+// Iteration i (slots of one MFMA each; the order is pinned by a scheduling
+// barrier per slot):
+//   slots  0-31: QK(i + 1)    slots 32-63: PV(i - 1), own keys' steps first
+//   slots  0-59: P'(i) = exp2(S(i)) * v_scale of the own keys
+//   slots 36-50: row maxima of S(i + 1), published before barrier B
+//   slot   20:   barrier A    slot 52: barrier B
+// Score and probability buffers alternate, so the loop is unrolled by two.  A
+// moved running max rescales O at the end of the next iteration, when PV of
+// the page before -- still relative to the old max -- is in it.
+//
+// K tiles live in a two-slot ring, V tiles in another, the scale planes in a
+// four-slot ring.  After A(i) nothing reads K(i + 1) any more (operand reads
+// run eight fragments ahead), so K(i + 3) is loaded into its slot between A(i)
+// and B(i); it is complete at B(i + 1), from where its first operands are
+// read.  After B(i) nothing reads V(i - 1), V(i + 1) is loaded between B(i)
+// and the end of the iteration and complete at A(i + 2).  At both barriers
+// the newest V and K group (8 + 9 pieces per wave) stay in flight.  P(i) is
+// written after B(i) and read by the partner after A(i + 1).  Page indices are
+// clamped to the segment: a clamped piece fills a slot that nothing reads any
+// more, or (V(-1)) one that is multiplied by P = 0.
+struct PW256 {
+  static constexpr int D = 256;
+  static constexpr int NW = 4, THREADS = 256, ROWS = 128;
+  // Tile image: K rows (64 x 528 B, as Tile<256>), v_scale[64] | v_zero[64]
+  // (one 1 KB piece), V^T rows of 128 B: 16-byte chunk c of row d at position
+  // c ^ ((d >> 1) & 7), so that 16 rows' reads of one chunk hit all banks.
+  static constexpr int KROW = 528, K_BYTES = 64 * KROW;
+  static constexpr int SC_OFF = K_BYTES;
+  static constexpr int V_OFF = SC_OFF + 1024;
+  static constexpr int V_BYTES = D * 128;
+  static constexpr int IMG = V_OFF + V_BYTES;
+  // LDS
+  static constexpr int L_V = 2 * K_BYTES;
+  static constexpr int L_SC = L_V + 2 * V_BYTES;
+  static constexpr int L_P = L_SC + 4 * 1024;
+  static constexpr int L_MAX = L_P + NW * 4096;
+  static constexpr int LDS = L_MAX + NW * 512;
+  static_assert(K_BYTES == 33 * 1024 && V_BYTES == 32 * 1024, "piece assignment of the DMAs");
+  static_assert(LDS <= 160 * 1024, "LDS");
+  static_assert(ROWS == Tile<256>::ROWS, "one block shape per head dim");
+};
+
+// Lane 16 r + E of each row r of 16 lanes, in all lanes of the row.
+template <int E>
+__device__ __forceinline__ float row_bcast(float x) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x150 + E, 0xf, 0xf, true));
+}
+
+__device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *smem, int h, int rb, int p_lo, int p_hi,
+                                                 PageOrder ord, float *part, int wv, int lane) {
+  constexpr int D = PW256::D, DS = D / 16;
+  const int n = p_hi - p_lo;
+  const int nrows = a.q_len * 6;
+  const int row0 = rb * PW256::ROWS + 64 * (wv >> 1);
+  const int half = wv & 1;
+  const int hh = lane / 32, r32 = lane % 32;
+
+  // DMAs.  K group of tile j (nine per wave): K pieces 8 wv .. + 7, then K 32
+  // (waves 0, 2) or the scale piece (waves 1, 3).  V group (eight): V pieces
+  // 8 wv .. + 7.
+  const uint32_t lane16 = 16 * lane;
+  auto tile_of = [&](int q) { return a.tiles + static_cast<int64_t>(ord.page(min(max(q, 0), n - 1))) * PW256::IMG; };
+  auto dma_k = [&](int q, int x) {
+    const char *src = tile_of(q);
+    if (x < 4) {
+      const int off = 8192 * wv + 2048 * x;
+      dma_piece_pair(src + off, lane16, (lds_t *)(smem + (q & 1) * PW256::K_BYTES + off));
+    } else {
+      const int dst = half ? PW256::L_SC + (q & 3) * 1024 : (q & 1) * PW256::K_BYTES + 32 * 1024;
+      dma_piece(src + 1024 * (32 + half), lane16, (lds_t *)(smem + dst));
+    }
+  };
+  auto dma_v = [&](int q, int x) {
+    const int off = 8192 * wv + 2048 * x;
+    dma_piece_pair(tile_of(q) + PW256::V_OFF + off, lane16, (lds_t *)(smem + PW256::L_V + (q & 1) * PW256::V_BYTES + off));
+  };
+#pragma unroll
+  for (int x = 0; x < 5; ++x) dma_k(0, x);
+#pragma unroll
+  for (int x = 0; x < 5; ++x) dma_k(1, x);
+#pragma unroll
+  for (int x = 0; x < 4; ++x) dma_v(-1, x);
+
+  // ---- query fragments of the pair's two row tiles and the row limits
+  v8h qf[2][DS];
+  int lim[2];
+  bool row_valid[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const int row = row0 + rt * 32 + r32;
+    row_valid[rt] = row < nrows;
+    const int tok = row_valid[rt] ? row / 6 : 0;
+    const int qh = h * 6 + (row_valid[rt] ? row % 6 : 0);
+    lim[rt] = row_valid[rt] ? a.seq_len - a.q_len + tok + 1 : 1;
+    const uint16_t *src = a.q + static_cast<int64_t>(tok) * a.q_tok_stride + static_cast<int64_t>(qh) * D + 8 * hh;
+    if (a.q_bf16) {
+#pragma unroll
+      for (int ds = 0; ds < DS; ++ds) {
+        const uint4 raw = row_valid[rt] ? *reinterpret_cast<const uint4 *>(src + 16 * ds) : make_uint4(0, 0, 0, 0);
+        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          qf[rt][ds][2 * e] = static_cast<_Float16>(__uint_as_float(w[e] << 16));
+          qf[rt][ds][2 * e + 1] = static_cast<_Float16>(__uint_as_float(w[e] & 0xFFFF0000u));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int ds = 0; ds < DS; ++ds) {
+        const uint4 raw = row_valid[rt] ? *reinterpret_cast<const uint4 *>(src + 16 * ds) : make_uint4(0, 0, 0, 0);
+        qf[rt][ds] = __builtin_bit_cast(v8h, raw);
+      }
+    }
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds) {
+      if (rt == 0)
+        asm volatile("" : "+a"(qf[rt][ds]));
+      else
+        asm volatile("" : "+v"(qf[rt][ds]));
+    }
+  }
+  const int full_pages = (a.seq_len - a.q_len + rb * PW256::ROWS / 6 + 1) / 64;
+
+  v16f O[2][4];       // dims 128 half + 32 dt ..
+  uint32_t pA[2][8], pB[2][8];  // own keys' P', packed fp16 pairs: key steps 2 half, 2 half + 1 in words 0-3, 4-7
+  uint32_t pX[2][8];  // the partner's
+  v16f sA[2], sB[2];
+  v16f minit[2];      // -m of the row (0 before its first visible key), the QK accumulators' start
+  float m_run[2], lsum[2], corr[2], alpha_o[2], mx[2];
+  float vs, vz;       // scale and zero point of key 8 (e / 4) + 4 hh + e % 4 of the own half, e = lane % 16
+  bool rescale_o = false;
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      O[rt][dt] = (v16f)0.f;
+      asm volatile("" : "+a"(O[rt][dt]));
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) pB[rt][e] = 0;
+    minit[rt] = (v16f)0.f;
+    m_run[rt] = -INFINITY;
+    lsum[rt] = corr[rt] = 0.f;
+    alpha_o[rt] = 1.f;
+  }
+
+  // LDS addresses: everything but a slot parity, a fragment index or the
+  // scale slot is per lane.
+  const char *kbase = smem + (32 * half + r32) * PW256::KROW + 16 * hh;
+  const char *vbase[4];  // key step of the second half's k-th group: own two, then the partner's two
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int c = 4 * (k < 2 ? half : 1 - half) + 2 * (k & 1) + hh;
+    vbase[k] = smem + PW256::L_V + (128 * half + r32) * 128 + ((c ^ ((r32 >> 1) & 7)) * 16);
+  }
+  char *const p_own = smem + PW256::L_P + 4096 * wv + 16 * lane;
+  const char *const p_partner = smem + PW256::L_P + 4096 * (wv ^ 1) + 16 * lane;
+  float2 *const max_own = reinterpret_cast<float2 *>(smem + PW256::L_MAX + 512 * wv) + lane;
+  const float2 *const max_partner = reinterpret_cast<const float2 *>(smem + PW256::L_MAX + 512 * (wv ^ 1)) + lane;
+  const int sc_lane = 4 * (32 * half + 8 * ((lane & 15) >> 2) + 4 * hh + (lane & 3));
+  auto k_frag = [&](int par, int f) -> v8h {
+    return *reinterpret_cast<const v8h *>(kbase + par * PW256::K_BYTES + 32 * f);
+  };
+  auto v_frag = [&](int par, int f) -> v8h {
+    return *reinterpret_cast<const v8h *>(vbase[f >> 2] + par * PW256::V_BYTES + 4096 * (f & 3));
+  };
+  auto frag4 = [](const uint32_t *w) -> v8h { return __builtin_bit_cast(v8h, make_uint4(w[0], w[1], w[2], w[3])); };
+  constexpr int AHEAD = 8;
+  v8h fr[AHEAD];
+
+  // Mask of page i's scores in the causal tail, then their maxima again.
+  auto mask = [&](int i, v16f (&S)[2]) {
+    const int p = ord.page(i);
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      mx[rt] = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        if (p * 64 + 32 * half + 8 * (e >> 2) + 4 * hh + (e & 3) >= lim[rt]) S[rt][e] = -INFINITY;
+        mx[rt] = fmaxf(mx[rt], S[rt][e]);
+      }
+    }
+  };
+  // The new running max of page i (`other`: the partner's maxima; both waves
+  // decide alike).  P' = p * v_scale has to stay a finite fp16: with every
+  // v_scale of the page at most 255 p may reach 2^8, else 2^2 (kThreshold).
+  auto fold_max = [&](int i, v16f (&S)[2], float2 other, float vs_lane) {
+    const float cm[2] = {fmaxf(mx[0], other.x), fmaxf(mx[1], other.y)};
+    const float lim_up = __ballot(vs_lane > 255.f) ? kThreshold : 8.f;
+    const float t0 = m_run[0] == -INFINITY ? -INFINITY : lim_up, t1 = m_run[1] == -INFINITY ? -INFINITY : lim_up;
+    if (__ballot(cm[0] > t0 || cm[1] > t1)) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        const float m_use = m_run[rt] == -INFINITY ? 0.f : m_run[rt];
+        auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(cm[rt]), __float_as_uint(cm[rt]), false, false);
+        const float rmx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) + m_use;
+        const float mnew = fmaxf(m_run[rt], rmx);
+        alpha_o[rt] = m_run[rt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[rt] - mnew);
+        m_run[rt] = mnew;
+        lsum[rt] *= alpha_o[rt];
+        corr[rt] *= alpha_o[rt];
+        const float m_new_use = mnew == -INFINITY ? 0.f : mnew;
+        minit[rt] = (v16f)(-m_new_use);
+        S[rt] -= m_new_use - m_use;
+      }
+      rescale_o = true;
+    }
+  };
+
+  // ---- prologue: S(0) from K(0), its running max, then K(2) over K(0) and V(0)
+  asm volatile("s_waitcnt vmcnt(17)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int f = 0; f < 16; ++f) {
+    const v8h kf = k_frag(0, f);
+    if (f == 0) {
+      mfma_score0(sA[0], kf, qf[0][f], minit[0]);
+      mfma_score0_v(sA[1], kf, qf[1][f], minit[1]);
+    } else {
+      mfma_score(sA[0], kf, qf[0][f]);
+      mfma_score_v(sA[1], kf, qf[1][f]);
+    }
+  }
+  mfma_settle();
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    mx[rt] = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) mx[rt] = fmaxf(mx[rt], sA[rt][e]);
+  }
+  if (ord.page(0) >= full_pages) mask(0, sA);
+  *max_own = make_float2(mx[0], mx[1]);
+#pragma unroll
+  for (int w = 0; w < 4; ++w) *reinterpret_cast<uint4 *>(p_own + 1024 * w) = make_uint4(0, 0, 0, 0);  // P(-1)
+  lds_barrier();
+#pragma unroll
+  for (int x = 0; x < 5; ++x) dma_k(2, x);
+#pragma unroll
+  for (int x = 0; x < 4; ++x) dma_v(0, x);
+  vs = *reinterpret_cast<const float *>(smem + PW256::L_SC + sc_lane);
+  vz = *reinterpret_cast<const float *>(smem + PW256::L_SC + 256 + sc_lane);
+  fold_max(0, sA, *max_partner, *reinterpret_cast<const float *>(smem + PW256::L_SC + 4 * lane));
+  rescale_o = false;  // O is zero
+  asm volatile("s_waitcnt vmcnt(25) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int f = 0; f < AHEAD; ++f) fr[f] = k_frag(1, f);
+
+  // Iteration i of parity `par`: sc = S(i), sn = S(i + 1); pp = P(i - 1), pn = P(i).
+  auto iteration = [&](int i, auto par_c, v16f (&sc)[2], v16f (&sn)[2], uint32_t (&pp)[2][8], uint32_t (&pn)[2][8]) {
+    constexpr int par = decltype(par_c)::value;
+    float pv0 = 0.f;
+    auto slot = [&](auto sl) {
+      constexpr int s = decltype(sl)::value;
+      constexpr int f = (s & 31) >> 1, rt = s & 1;
+      if constexpr (s < 32) {
+        if constexpr (f == 0 && rt == 0) mfma_score0(sn[0], fr[f % AHEAD], qf[0][f], minit[0]);
+        if constexpr (f == 0 && rt == 1) mfma_score0_v(sn[1], fr[f % AHEAD], qf[1][f], minit[1]);
+        if constexpr (f > 0 && rt == 0) mfma_score(sn[0], fr[f % AHEAD], qf[0][f]);
+        if constexpr (f > 0 && rt == 1) mfma_score_v(sn[1], fr[f % AHEAD], qf[1][f]);
+      } else {
+        constexpr int k = f >> 2;
+        mfma_out(O[rt][f & 3], fr[f % AHEAD], k < 2 ? frag4(&pp[rt][4 * k]) : frag4(&pX[rt][4 * (k - 2)]));
+      }
+      // Operand reads: this half's fragments 8-15 in its first 16 slots, the
+      // next half's 0-7 from the barrier (local slot 20) on.
+      constexpr int ls = s & 31;
+      auto next_frag = [&](int g) { fr[g] = s < 32 ? v_frag(1 - par, g) : k_frag(par, g); };
+      if constexpr (ls < 16 && rt == 1) fr[f] = s < 32 ? k_frag(1 - par, f + 8) : v_frag(1 - par, f + 8);
+      if constexpr (ls == 20) {
+        next_frag(0);
+        next_frag(1);
+      }
+      if constexpr (ls > 20 && rt == 1) next_frag((ls - 17) >> 1);
+      // P'(i) of the own keys: 32 scores of the lane over slots 0-59.
+      constexpr int x0 = s < 60 ? s * 32 / 60 : 32, x1 = s < 60 ? (s + 1) * 32 / 60 : 32;
+      if constexpr (x1 > x0) {
+        constexpr int r = (x0 >> 3) & 1, st = x0 >> 4, j = x0 & 7, e = 8 * st + j;
+        const float pr = __builtin_amdgcn_exp2f(sc[r][e]);
+        lsum[r] += pr;
+        const float pv = pr * row_bcast<e>(vs);
+        corr[r] = fmaf(row_bcast<e>(vz), pv, corr[r]);
+        asm volatile("" : "+v"(lsum[r]), "+v"(corr[r]));
+        if constexpr (j & 1) {
+          const v2h two = {static_cast<_Float16>(pv0), static_cast<_Float16>(pv)};
+          pn[r][4 * st + (j >> 1)] = __builtin_bit_cast(uint32_t, two);
+          asm volatile("" : "+v"(pn[r][4 * st + (j >> 1)]));  // computed here, not where it is used
+        } else {
+          pv0 = pv;
+        }
+      }
+      // Maxima of S(i + 1): 16 pairs over slots 36-50.
+      if constexpr (s >= 36 && s < 51) {
+        constexpr int k0 = (s - 36) * 16 / 15, k1 = (s - 35) * 16 / 15;
+#pragma unroll
+        for (int k = k0; k < k1; ++k) {
+          const int r = k & 1, e = 2 * (k >> 1);
+          mx[r] = fmaxf(fmaxf(mx[r], sn[r][e]), sn[r][e + 1]);
+          asm volatile("" : "+v"(mx[r]));
+        }
+      }
+      // The partner's P(i - 1), after barrier A; the own P(i), after barrier B.
+      if constexpr (s >= 22 && s < 30 && rt == 0) {
+        constexpr int w = (s - 22) >> 1;  // (row tile, key step)
+        const uint4 x = *reinterpret_cast<const uint4 *>(p_partner + 1024 * w);
+        uint32_t *d = &pX[w >> 1][4 * (w & 1)];
+        d[0] = x.x, d[1] = x.y, d[2] = x.z, d[3] = x.w;
+      }
+      if constexpr (s == 53 || s == 55 || s == 57 || s == 62) {
+        // completed in the order (key step, row tile)
+        constexpr int w = s == 53 ? 0 : s == 55 ? 2 : s == 57 ? 1 : 3;
+        const uint32_t *d = &pn[w >> 1][4 * (w & 1)];
+        *reinterpret_cast<uint4 *>(p_own + 1024 * w) = make_uint4(d[0], d[1], d[2], d[3]);
+      }
+      if constexpr (s >= 22 && s < 52 && (s - 22) % 6 == 0) dma_k(i + 3, (s - 22) / 6);
+      if constexpr (s >= 53 && (s - 53) % 3 == 0) dma_v(i + 1, (s - 53) / 3);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    mx[0] = mx[1] = -INFINITY;
+    static_for<20>([&](auto sl) { slot(sl); });
+    asm volatile("s_waitcnt vmcnt(17) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    static_for<31>([&](auto sl) { slot(std::integral_constant<int, 20 + decltype(sl)::value>{}); });
+    const bool more = i + 1 < n;
+    if (__builtin_expect(more && ord.page(i + 1) >= full_pages, 0)) mask(i + 1, sn);
+    *max_own = make_float2(mx[0], mx[1]);
+    slot(std::integral_constant<int, 51>{});
+    asm volatile("s_waitcnt vmcnt(17) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    slot(std::integral_constant<int, 52>{});
+    const char *scp = smem + PW256::L_SC + ((i + 1) & 3) * 1024;
+    const float2 other = *max_partner;
+    const float vs_next = *reinterpret_cast<const float *>(scp + sc_lane);
+    const float vz_next = *reinterpret_cast<const float *>(scp + 256 + sc_lane);
+    const float vs_lane = *reinterpret_cast<const float *>(scp + 4 * lane);
+    static_for<11>([&](auto sl) { slot(std::integral_constant<int, 53 + decltype(sl)::value>{}); });
+    vs = vs_next;
+    vz = vz_next;
+    if (__builtin_expect(rescale_o, 0)) {
+      mfma_settle();
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc_scale(O[rt][dt], e, alpha_o[rt]);
+      rescale_o = false;
+    }
+    if (more) fold_max(i + 1, sn, other, vs_lane);
+  };
+  bool odd = false;  // P(n - 1) is in pA unless n is even
+  for (int i = 0; i < n; i += 2) {
+    iteration(i, std::integral_constant<int, 0>{}, sA, sB, pB, pA);
+    odd = true;
+    if (i + 1 >= n) break;
+    iteration(i + 1, std::integral_constant<int, 1>{}, sB, sA, pA, pB);
+    odd = false;
+  }
+  mfma_settle();
+  // ---- PV(n - 1): all V in place, the partner's P(n - 1)
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const uint4 x = *reinterpret_cast<const uint4 *>(p_partner + 1024 * w);
+    uint32_t *d = &pX[w >> 1][4 * (w & 1)];
+    d[0] = x.x, d[1] = x.y, d[2] = x.z, d[3] = x.w;
+  }
+  if (odd) {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) pB[rt][e] = pA[rt][e];
+  }
+  const int last_v = ((n - 1) & 1) * PW256::V_BYTES;
+#pragma unroll
+  for (int f = 0; f < 16; ++f) {
+    const v8h vf = *reinterpret_cast<const v8h *>(vbase[f >> 2] + last_v + 4096 * (f & 3));
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+      mfma_out(O[rt][f & 3], vf, f < 8 ? frag4(&pB[rt][4 * (f >> 2)]) : frag4(&pX[rt][4 * ((f >> 2) - 2)]));
+  }
+  // Row sums and zero-point terms of both halves of the keys.
+  float l[2], cz[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    auto a1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum[rt]), __float_as_uint(lsum[rt]), false, false);
+    l[rt] = __uint_as_float(a1[0]) + __uint_as_float(a1[1]);
+    auto a2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(corr[rt]), __float_as_uint(corr[rt]), false, false);
+    cz[rt] = __uint_as_float(a2[0]) + __uint_as_float(a2[1]);
+  }
+  lds_barrier();  // the partner has read P(n - 1)
+  *reinterpret_cast<float4 *>(p_own) = make_float4(l[0], l[1], cz[0], cz[1]);
+  lds_barrier();
+  const float4 oth = *reinterpret_cast<const float4 *>(p_partner);
+  l[0] += oth.x;
+  l[1] += oth.y;
+  cz[0] += oth.z;
+  cz[1] += oth.w;
+  lds_barrier();  // read before the next segment overwrites it
+  mfma_settle();
+
+  // ---- finalize: O = (acc * 2^24|2^20 - corr) / l, dims 128 half ..
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const int row = row0 + rt * 32 + r32;
+    if (part) {
+      const int lr = row - rb * PW256::ROWS;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v4f o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = O[rt][dt][4 * j + e] * ((e & 1) ? 1048576.f : 16777216.f) - cz[rt];
+          *reinterpret_cast<v4f *>(part + lr * D + 128 * half + 32 * dt + 8 * j + 4 * hh) = o;
+        }
+      if (half == 0 && hh == 0) {
+        part[PW256::ROWS * D + lr] = m_run[rt];
+        part[PW256::ROWS * D + PW256::ROWS + lr] = l[rt];
+      }
+    } else if (row_valid[rt]) {
+      const float inv = l[rt] > 0.f ? 1.f / l[rt] : 0.f;
+      const int tok = row / 6, qh = h * 6 + row % 6;
+      const int64_t ob =
+          static_cast<int64_t>(tok) * a.out_tok_stride + static_cast<int64_t>(qh) * D + 128 * half + 4 * hh;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v4f o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = (O[rt][dt][4 * j + e] * ((e & 1) ? 1048576.f : 16777216.f) - cz[rt]) * inv;
+          store_out4(a.out, a.out_dtype, ob + 32 * dt + 8 * j, o);
+        }
+    }
+  }
+}
+
+// Attention of one KV head over its tile images.
+__global__ __attribute__((amdgpu_flat_work_group_size(PW256::THREADS, PW256::THREADS), amdgpu_waves_per_eu(1, 1))) void
+prefill_tiles256_kernel(PrefillArgs a) {
+  __shared__ __attribute__((aligned(16))) char smem[PW256::LDS];
+  const int w = blockIdx.x;
+  const int v = a.xcd_perm ? (w % 8) * (a.grid / 8) + w / 8 : w;
+  const int s0 = range_start(a, v), s1 = range_start(a, v + 1);
+  if (s0 >= s1) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int lane = threadIdx.x % 64;
+  for (int e = s1; e > s0;) {
+    const TileSegment g = last_segment(a, s0, s1, e, lane);
+    float *part = nullptr;
+    if (!g.whole) part = a.ws + (static_cast<int64_t>(v) * 2 + g.slot) * PW256::ROWS * (PW256::D + 2);
+    run_segment_pair(a, smem, a.head0 + g.hl, g.rb, g.p_lo, g.p_hi, g.order, part, wave, lane);
+    e -= g.p_hi - g.p_lo;
+  }
+}
+
 template <int D, bool PRE>
 __global__ __attribute__((amdgpu_flat_work_group_size(Tile<D>::THREADS, Tile<D>::THREADS),
                           amdgpu_waves_per_eu(Tile<D>::WPE, Tile<D>::WPE))) void
 prefill_kernel(PrefillArgs a) {
   using T = Tile<D>;
-  constexpr int LDS_BYTES = D == 128 ? PP::LDS : (PRE ? 2 * T::TBUF : 2 * T::BUF + T::STAGE);
+  static_assert(D == 128 || !PRE, "head dim 256 over tile images: prefill_tiles256_kernel");
+  constexpr int LDS_BYTES = D == 128 ? PP::LDS : 2 * T::BUF + T::STAGE;
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
   const int w = blockIdx.x;
   const int v = a.xcd_perm ? (w % 8) * (a.grid / 8) + w / 8 : w;
@@ -1174,7 +1743,7 @@ prefill_kernel(PrefillArgs a) {
     if constexpr (D == 128)
       run_segment_pp<PRE>(a, smem, h, rb, p_lo, p_hi, part, tid, wave, lane);
     else
-      run_segment<D, PRE>(a, smem, h, rb, p_lo, p_hi, part, tid, wave, lane);
+      run_segment<D>(a, smem, h, rb, p_lo, p_hi, part, tid, wave, lane);
     s += p_hi - p_lo;
     first = false;
   }
@@ -1232,19 +1801,26 @@ __global__ __launch_bounds__(256) void prefill_convert_kernel(PrefillArgs a, cha
 // (TBUF bytes: the tail past BUF carries staged codes nothing reads).
 __global__ __launch_bounds__(256) void prefill_convert256_kernel(PrefillArgs a, char *tiles, int h) {
   using T = Tile<256>;
-  static_assert(T::THREADS == 256 && T::TBUF <= T::BUF + T::STAGE, "one page per work-group of four waves");
+  static_assert(T::THREADS == 256 && T::KROW == PW256::KROW, "one page per work-group of four waves");
   __shared__ __attribute__((aligned(16))) char smem[T::BUF + T::STAGE];
   const int p = blockIdx.x, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
   stage_page<256>(a, p, h, wave, lane, (lds_t *)(smem + T::BUF), (lds_t *)(smem + T::S_OFF));
   wait_dma();
   __syncthreads();
-  convert_page<256>(a, p, smem + T::BUF, smem, tid);
+  convert_page<256, true>(a, p, smem + T::BUF, smem, tid);
   __syncthreads();
-  char *dst = tiles + static_cast<int64_t>(p) * T::TBUF;
+  char *dst = tiles + static_cast<int64_t>(p) * PW256::IMG;
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  for (int o = 16 * tid; o < T::TBUF; o += 16 * T::THREADS)
+  for (int o = 16 * tid; o < PW256::K_BYTES; o += 16 * T::THREADS)
     tile_store<true>(dst + o, *reinterpret_cast<const u32x4 *>(smem + o));
+  if (tid < 32) tile_store<true>(dst + PW256::SC_OFF + 16 * tid, *reinterpret_cast<const u32x4 *>(smem + T::S_OFF + 256 + 16 * tid));
+  for (int o = tid; o < PW256::V_BYTES / 16; o += T::THREADS) {
+    const int row = o >> 3, c = (o & 7) ^ ((row >> 1) & 7);
+    const char *src = smem + T::V_OFF + row * T::VROW + 16 * c;
+    const uint2 lo = *reinterpret_cast<const uint2 *>(src), hi = *reinterpret_cast<const uint2 *>(src + 8);
+    tile_store<true>(dst + PW256::V_OFF + 16 * o, (u32x4){lo.x, lo.y, hi.x, hi.y});
+  }
 }
 
 // Finishes the blocks split between work-groups: kMergeSplit work-groups of
@@ -1471,7 +2047,7 @@ bool tiles_pay_off(int64_t nbh, int64_t npages, int head_dim) {
 }
 
 bool use_tiles(const PrefillPlan &pl, int /*head_dim*/) { return pl.tiles; }
-int64_t tile_stride(int head_dim) { return head_dim == 128 ? PP::BUF : Tile<256>::TBUF; }
+int64_t tile_stride(int head_dim) { return head_dim == 128 ? PP::BUF : PW256::IMG; }
 
 // Persistent work-groups for a launch of `steps` page steps: one per CU, each
 // with at least kMinSteps steps (a work-group's fixed work -- its query rows,
@@ -1665,7 +2241,7 @@ extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stri
         prefill_merge_kernel<128><<<dim3(static_cast<unsigned>(pl.nbh * kMergeSplit)), dim3(kMergeThreads), 0, s>>>(a);
       } else {
         prefill_convert256_kernel<<<dim3(npages), dim3(256), 0, s>>>(a, tiles, h);
-        prefill_kernel<256, true><<<dim3(static_cast<unsigned>(a.grid)), dim3(Tile<256>::THREADS), 0, s>>>(a);
+        prefill_tiles256_kernel<<<dim3(static_cast<unsigned>(a.grid)), dim3(PW256::THREADS), 0, s>>>(a);
         prefill_merge_kernel<256><<<dim3(static_cast<unsigned>(pl.nbh * kMergeSplit)), dim3(kMergeThreads), 0, s>>>(a);
       }
       const int rc = launch_status("k8v4_prefill_paged");

@@ -1,0 +1,91 @@
+"""Prefill over tile images: segment edges, row remainders and the running max (GPU).
+
+The kernels that multiply from pre-dequantized page images cut the row blocks
+into segments of any length from one page up, visit a segment's pages in a
+rotated order and run several pages at once, so the cases below have segments
+of one, two and more pages, a last block with few rows, a last page with few
+keys, and scores that keep rising so that the running max moves late and often.
+"""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_cases import DEV, Cache, assert_close, fill_sequence, random_tables, seeded_normal
+from k8v4_v030.layout import PAGE, PageLayout
+from k8v4_v030.prefill import hip_prefill
+from oracle import torch_cpu
+from oracle.paged import Geometry
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(cache, q, row, seq_len):
+    out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=DEV)
+    hip_prefill(q.to(DEV), cache.views, row.to(device=DEV, dtype=torch.int32), seq_len, 1,
+                1.0 / math.sqrt(q.shape[2]), out=out)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def _want(cache, q, row, seq_len):
+    lay = cache.layout
+    views = torch_cpu.region_views(torch.from_numpy(cache.blob().copy()), Geometry(lay.hkv, lay.head_dim))
+    return torch_cpu.prefill(views, q, row.long(), seq_len, 1.0 / math.sqrt(lay.head_dim)).numpy()
+
+
+@pytest.mark.parametrize("hkv,d,q_len,seq_len", [
+    # whole prompts: 27 steps a work-group over blocks of 1 to 68 pages
+    (2, 256, 4300, 4300), (4, 256, 2817, 3901),
+    # one key in the last page, six rows in the last block
+    (2, 256, 2049, 16385),
+    (4, 128, 129, 129), (2, 128, 171, 65), (4, 128, 683, 1985), (2, 128, 1999, 1999),
+])
+def test_segments_of_every_length(gpu_ops, hkv, d, q_len, seq_len):
+    seq_len = max(q_len, seq_len)
+    print("prefill tiles hkv=%d d=%d q=%d seq=%d" % (hkv, d, q_len, seq_len), flush=True)
+    assert gpu_ops.prefill_uses_tiles(seq_len, q_len, hkv, d)
+    lay = PageLayout(hkv, d)
+    gen = torch.Generator().manual_seed(q_len + seq_len + hkv + d)
+    pages = -(-seq_len // PAGE)
+    cache = Cache(pages + 3, lay)
+    table = random_tables(gen, [seq_len], pages + 3)
+    fill_sequence(gpu_ops, cache, gen, table[0], seq_len)
+    q = seeded_normal(gen, (q_len, lay.hq, d))
+    assert_close(_run(cache, q, table[0], seq_len), _want(cache, q, table[0], seq_len), what="tiles")
+
+
+@pytest.mark.parametrize("vmax", [65504.0, 1.0])
+@pytest.mark.parametrize("d,q_len,seq_len", [(256, 2100, 8192), (128, 200, 8192)])
+def test_running_max_moves_late_and_often(gpu_ops, d, q_len, seq_len, vmax):
+    """Each 32-token chunk scores 0.25 (log2 units) above the one before, with
+    V rows of +-vmax whose sign alternates from chunk to chunk: with the widest
+    V an fp16 row can hold P' = p * v_scale overflows past a lag of 2.9, with a
+    small one the lag may grow to 8.
+
+    Tolerance: scores reach 64 log2 units, the keys of the tile images are
+    rounded to fp16 once (2^-12 relative), so two neighbouring chunks' weights
+    may shift against each other by 2 * 64 * 2^-12 log2 units = 2.2 %."""
+    print("prefill rising d=%d q=%d vmax=%g" % (d, q_len, vmax), flush=True)
+    lay = PageLayout(2, d)
+    gen = torch.Generator().manual_seed(d + q_len)
+    pages = seq_len // PAGE
+    cache = Cache(pages + 3, lay)
+    table = random_tables(gen, [seq_len], pages + 3)
+    t = torch.arange(seq_len)
+    per_c = math.sqrt(d) * 1.4426950408889634  # log2 score of a ones query per unit of c
+    c = (t // 32).float() * (0.25 / per_c)
+    k = (c[:, None, None] * torch.ones((seq_len, 2, d))).to(torch.float16)
+    sign = 1.0 - 2.0 * ((t // 32) % 2).float()
+    v = (sign[:, None, None] * torch.full((seq_len, 2, d), vmax)).to(torch.float16)
+    v[:, :, 1::2] = -v[:, :, 1::2]
+    slots = (table[0].long()[t // PAGE] * PAGE + t % PAGE).to(DEV)
+    cache.store(gpu_ops, k.to(DEV), v.to(DEV), slots)
+    q = torch.ones((q_len, 12, d), dtype=torch.float16)
+    assert gpu_ops.prefill_uses_tiles(seq_len, q_len, 2, d)
+    want = _want(cache, q, table[0], seq_len)
+    assert np.abs(want).max() > 0.05 * vmax
+    assert_close(_run(cache, q, table[0], seq_len), want, atol=0.022 * vmax, rtol=1e-2, what="rising scores")
