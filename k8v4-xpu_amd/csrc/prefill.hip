@@ -88,7 +88,8 @@ struct PrefillArgs {
   int xcd_perm;  // map ids so the work-groups of one XCD take adjacent work (grid % 8 == 0)
   float *ws;     // partial states: [grid][2][rows][D + 2] floats
   int head0;     // KV head of step 0 (a launch covers heads head0 .. head0 + total / tper - 1)
-  const char *tiles;  // dequantized tiles of head head0, [page][PP::BUF] (D = 128) or [page][PW256::IMG] bytes (null: convert in-kernel)
+  const char *tiles;  // dequantized tiles from head head0 on, [head][page][PP::BUF] (D = 128) or [page][PW256::IMG] bytes (null: convert in-kernel)
+  int64_t tile_head;  // bytes of one head's tiles
   void *out;
   int out_dtype;
   int64_t out_tok_stride;  // elements
@@ -845,7 +846,7 @@ __device__ __forceinline__ void run_segment_pp(const PrefillArgs &a, char *smem,
   // DMA pieces of one tile (1 KB each, 35 per tile): piece k belongs to group
   // k % 2, wave (k / 2) % 4 of it.
   static_assert(PP::BUF % 1024 == 0 && 4 * PP::BUF <= PP::LDS, "tile pieces and four-slot ring");
-  const char *tsrc = PRE ? a.tiles + static_cast<int64_t>(p_lo) * PP::BUF : nullptr;
+  const char *tsrc = PRE ? a.tiles + (h - a.head0) * a.tile_head + static_cast<int64_t>(p_lo) * PP::BUF : nullptr;
   auto tile_dma = [&](int q) {
 #pragma unroll
     for (int j = 0; j < 5; ++j) {
@@ -1316,7 +1317,8 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
   // (waves 0, 2) or the scale piece (waves 1, 3).  V group (eight): V pieces
   // 8 wv .. + 7.
   const uint32_t lane16 = 16 * lane;
-  auto tile_of = [&](int q) { return a.tiles + static_cast<int64_t>(ord.page(min(max(q, 0), n - 1))) * PW256::IMG; };
+  const char *tiles = a.tiles + (h - a.head0) * a.tile_head;
+  auto tile_of = [&](int q) { return tiles + static_cast<int64_t>(ord.page(min(max(q, 0), n - 1))) * PW256::IMG; };
   auto dma_k = [&](int q, int x) {
     const char *src = tile_of(q);
     if (x < 4) {
@@ -1689,7 +1691,7 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
   }
 }
 
-// Attention of one KV head over its tile images.
+// Attention of KV heads over their tile images.
 __global__ __attribute__((amdgpu_flat_work_group_size(PW256::THREADS, PW256::THREADS), amdgpu_waves_per_eu(1, 1))) void
 prefill_tiles256_kernel(PrefillArgs a) {
   __shared__ __attribute__((aligned(16))) char smem[PW256::LDS];
@@ -1749,18 +1751,18 @@ prefill_kernel(PrefillArgs a) {
   }
 }
 
-// Dequantizes every page of KV head h once into its tile image (the LDS
-// layout of run_segment_pp's ring): one work-group of 256 threads per page.
+// Dequantizes every page of a KV head (blockIdx.y) once into its tile image (the
+// LDS layout of run_segment_pp's ring): one work-group of 256 threads per page.
 // The page's V codes and scale planes are staged in LDS with coalesced loads
 // in the order the in-kernel conversion stages them; then each thread
 // dequantizes two K chunks (read directly) and two V items with the same
 // arithmetic as the in-kernel conversion.
-__global__ __launch_bounds__(256) void prefill_convert_kernel(PrefillArgs a, char *tiles, int h) {
+__global__ __launch_bounds__(256) void prefill_convert_kernel(PrefillArgs a, char *tiles) {
   constexpr int D = PP::D;
   __shared__ __attribute__((aligned(16))) char st[PP::STAGE];
-  const int p = blockIdx.x, t = threadIdx.x;
+  const int p = blockIdx.x, h = a.head0 + blockIdx.y, t = threadIdx.x;
   const int64_t phys = page_of(a, p);
-  char *buf = tiles + static_cast<int64_t>(p) * PP::BUF;
+  char *buf = tiles + blockIdx.y * a.tile_head + static_cast<int64_t>(p) * PP::BUF;
   const char *kb = reinterpret_cast<const char *>(a.k_cache) + phys * a.k_ps + h * D;
   const char *vb = reinterpret_cast<const char *>(a.v_cache) + phys * a.v_ps + h * (D / 2);
   const int64_t krow = static_cast<int64_t>(a.hkv) * D, vrow = static_cast<int64_t>(a.hkv) * (D / 2);
@@ -1794,23 +1796,23 @@ __global__ __launch_bounds__(256) void prefill_convert_kernel(PrefillArgs a, cha
   }
 }
 
-// D = 256: every page of KV head h dequantized once into its tile image (the
+// D = 256: every page of a KV head dequantized once into its tile image (the
 // LDS layout run_segment multiplies from), one work-group of four waves per
 // page: the page is staged and converted exactly as the attention kernel
 // does in place, then the image leaves LDS with nontemporal 16-byte stores
 // (TBUF bytes: the tail past BUF carries staged codes nothing reads).
-__global__ __launch_bounds__(256) void prefill_convert256_kernel(PrefillArgs a, char *tiles, int h) {
+__global__ __launch_bounds__(256) void prefill_convert256_kernel(PrefillArgs a, char *tiles) {
   using T = Tile<256>;
   static_assert(T::THREADS == 256 && T::KROW == PW256::KROW, "one page per work-group of four waves");
   __shared__ __attribute__((aligned(16))) char smem[T::BUF + T::STAGE];
-  const int p = blockIdx.x, tid = threadIdx.x;
+  const int p = blockIdx.x, h = a.head0 + blockIdx.y, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
   stage_page<256>(a, p, h, wave, lane, (lds_t *)(smem + T::BUF), (lds_t *)(smem + T::S_OFF));
   wait_dma();
   __syncthreads();
   convert_page<256, true>(a, p, smem + T::BUF, smem, tid);
   __syncthreads();
-  char *dst = tiles + static_cast<int64_t>(p) * PW256::IMG;
+  char *dst = tiles + blockIdx.y * a.tile_head + static_cast<int64_t>(p) * PW256::IMG;
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   for (int o = 16 * tid; o < PW256::K_BYTES; o += 16 * T::THREADS)
     tile_store<true>(dst + o, *reinterpret_cast<const u32x4 *>(smem + o));
@@ -2022,6 +2024,7 @@ namespace {
 struct PrefillPlan {
   int nbh, tper, total, grid;
   bool tiles;  // pages dequantized once per KV head into tile images
+  int heads;   // tiles: KV heads per launch
 };
 
 // Fewest page steps per persistent work-group when a call has few (one
@@ -2046,7 +2049,6 @@ bool tiles_pay_off(int64_t nbh, int64_t npages, int head_dim) {
   return head_dim == 128 || (9 * nbh - 62) * npages > 58600;
 }
 
-bool use_tiles(const PrefillPlan &pl, int /*head_dim*/) { return pl.tiles; }
 int64_t tile_stride(int head_dim) { return head_dim == 128 ? PP::BUF : PW256::IMG; }
 
 // Persistent work-groups for a launch of `steps` page steps: one per CU, each
@@ -2057,6 +2059,21 @@ int64_t persistent_grid(int64_t steps) {
   int64_t grid = std::min<int64_t>(static_cast<int64_t>(device_cus()), std::max<int64_t>(1, steps / kMinSteps));
   if (grid >= 8) grid -= grid % 8;
   return grid;
+}
+
+// KV heads that share one launch over their tile images: as many as keep the
+// launch's images within kTileSetBytes (half of the 256 MB MALL), at least
+// one.  A launch over one head of a short context leaves a work-group a few
+// page steps, and its ramp, tail and merge outweigh them: 1,999 tokens with
+// nothing before them, 4 heads of 128 dims: 232 us as four launches, 100 us as
+// one.  4,224 tokens over 131,072, whose images are 76 MB a head: 6,448 us
+// with one head a launch, 6,391 with two, 6,648 with four (past the MALL).
+constexpr int64_t kTileSetBytes = int64_t(128) << 20;
+int64_t tile_set_pages(int head_dim) { return kTileSetBytes / tile_stride(head_dim); }
+int heads_per_launch(int64_t npages, int hkv, int head_dim) {
+  const int64_t most = std::max<int64_t>(1, std::min<int64_t>(hkv, tile_set_pages(head_dim) / npages));
+  const int64_t launches = (hkv + most - 1) / most;
+  return static_cast<int>((hkv + launches - 1) / launches);  // 2 + 2 rather than 3 + 1
 }
 
 // Host mirror of the device schedule; false if the call is too large for it.
@@ -2074,9 +2091,10 @@ bool plan_prefill(int64_t seq_len, int64_t q_len, int hkv, int head_dim, Prefill
   pl.tper = static_cast<int>(tper);
   pl.total = static_cast<int>(total);
   pl.tiles = tiles_pay_off(nbh, (seq_len + kPage - 1) / kPage, head_dim);
-  // The grid of the launch that runs: one per KV head over its tper steps
-  // with tile images, else one over all heads.
-  pl.grid = static_cast<int>(persistent_grid(use_tiles(pl, head_dim) ? tper : total));
+  // The grid of the launch that runs: with tile images over the steps of
+  // pl.heads KV heads, else over all heads.
+  pl.heads = pl.tiles ? heads_per_launch((seq_len + kPage - 1) / kPage, hkv, head_dim) : hkv;
+  pl.grid = static_cast<int>(persistent_grid(tper * pl.heads));
   return true;
 }
 
@@ -2084,13 +2102,28 @@ int64_t partial_bytes(int grid, int head_dim) {
   return static_cast<int64_t>(grid) * 2 * rows_per_block(head_dim) * (head_dim + 2) * 4;
 }
 
-// Workspace: partial states, then (tiles) one head's tile images, 256-byte aligned.
+// Workspace: partial states, then (tiles) the tile images of a launch's heads, 256-byte aligned.
 int64_t tiles_offset(const PrefillPlan &pl, int head_dim) { return (partial_bytes(pl.grid, head_dim) + 255) / 256 * 256; }
 int64_t workspace_need(const PrefillPlan &pl, int64_t seq_len, int head_dim) {
-  if (!use_tiles(pl, head_dim)) return partial_bytes(pl.grid, head_dim);
-  return tiles_offset(pl, head_dim) + (seq_len + kPage - 1) / kPage * tile_stride(head_dim);
+  if (!pl.tiles) return partial_bytes(pl.grid, head_dim);
+  return tiles_offset(pl, head_dim) + pl.heads * ((seq_len + kPage - 1) / kPage) * tile_stride(head_dim);
 }
-
+// What a workspace is sized for: also every shorter context of the same call
+// (which may take more heads a launch: up to tile_set_pages of images).
+int64_t workspace_size(const PrefillPlan &pl, int64_t seq_len, int hkv, int head_dim) {
+  if (!pl.tiles) return partial_bytes(pl.grid, head_dim);
+  const int64_t npages = (seq_len + kPage - 1) / kPage;
+  const int64_t pages = std::min(hkv * npages, std::max(npages, tile_set_pages(head_dim)));
+  return (partial_bytes(static_cast<int>(persistent_grid(static_cast<int64_t>(pl.tper) * hkv)), head_dim) + 255) / 256 * 256 +
+         pages * tile_stride(head_dim);
+}
+// Fewer heads a launch, down to one, until the call fits `bytes`.
+void fit_workspace(PrefillPlan &pl, int64_t seq_len, int head_dim, int64_t bytes) {
+  while (pl.tiles && pl.heads > 1 && workspace_need(pl, seq_len, head_dim) > bytes) {
+    --pl.heads;
+    pl.grid = static_cast<int>(persistent_grid(static_cast<int64_t>(pl.tper) * pl.heads));
+  }
+}
 
 // Argument checks shared by the single-sequence and batched prefill entries.
 int check_prefill_args(const void *q, int q_dtype, int64_t q_tok_stride, const int8_t *k_cache, const float *k_scale,
@@ -2160,7 +2193,7 @@ extern "C" int64_t k8v4_prefill_workspace_bytes(int64_t seq_len, int64_t q_len, 
   if (q_len == 0) return 0;
   PrefillPlan pl;
   if (!plan_prefill(seq_len, q_len, hkv, head_dim, pl)) return -1;
-  return workspace_need(pl, seq_len, head_dim);
+  return workspace_size(pl, seq_len, hkv, head_dim);
 }
 
 extern "C" int k8v4_prefill_uses_tiles(int64_t seq_len, int64_t q_len, int hkv, int head_dim) {
@@ -2169,7 +2202,7 @@ extern "C" int k8v4_prefill_uses_tiles(int64_t seq_len, int64_t q_len, int hkv, 
   if (q_len == 0) return 0;
   PrefillPlan pl;
   if (!plan_prefill(seq_len, q_len, hkv, head_dim, pl)) return -1;
-  return use_tiles(pl, head_dim) ? 1 : 0;
+  return pl.tiles ? 1 : 0;
 }
 
 extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stride, const int8_t *k_cache,
@@ -2208,6 +2241,7 @@ extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stri
   PrefillPlan pl;
   K8V4_REQUIRE(plan_prefill(seq_len, q_len, hkv, head_dim, pl), "prefill too large for one call (q_len %lld, seq_len %lld)",
                static_cast<long long>(q_len), static_cast<long long>(seq_len));
+  fit_workspace(pl, seq_len, head_dim, workspace_bytes);
   const int64_t need = workspace_need(pl, seq_len, head_dim);
   K8V4_REQUIRE(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
                "prefill workspace must be a 16-byte aligned device buffer");
@@ -2226,23 +2260,29 @@ extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stri
   a.head0 = 0;
   a.tiles = nullptr;
   auto s = static_cast<hipStream_t>(stream);
-  if (use_tiles(pl, head_dim)) {
-    // One KV head at a time: its pages dequantized once into the workspace,
-    // then all row blocks of the head over them, then their merge.
+  if (pl.tiles) {
+    // pl.heads KV heads at a time: their pages dequantized once into the
+    // workspace, then all row blocks of those heads over them, then their merge.
     char *tiles = static_cast<char *>(workspace) + tiles_offset(pl, head_dim);
     const unsigned npages = static_cast<unsigned>((seq_len + kPage - 1) / kPage);
-    a.total = pl.tper;
     a.tiles = tiles;
-    for (int h = 0; h < hkv; ++h) {
+    a.tile_head = static_cast<int64_t>(npages) * tile_stride(head_dim);
+    for (int h = 0; h < hkv; h += pl.heads) {
+      const int heads = std::min(pl.heads, hkv - h);
       a.head0 = h;
+      a.total = pl.tper * heads;
+      a.grid = static_cast<int>(persistent_grid(a.total));
+      a.xcd_perm = a.grid % 8 == 0 ? 1 : 0;
+      const dim3 cgrid(npages, static_cast<unsigned>(heads)), grid(static_cast<unsigned>(a.grid));
+      const dim3 mgrid(static_cast<unsigned>(pl.nbh * heads * kMergeSplit));
       if (head_dim == 128) {
-        prefill_convert_kernel<<<dim3(npages), dim3(256), 0, s>>>(a, tiles, h);
-        prefill_kernel<128, true><<<dim3(static_cast<unsigned>(a.grid)), dim3(PP::THREADS), 0, s>>>(a);
-        prefill_merge_kernel<128><<<dim3(static_cast<unsigned>(pl.nbh * kMergeSplit)), dim3(kMergeThreads), 0, s>>>(a);
+        prefill_convert_kernel<<<cgrid, dim3(256), 0, s>>>(a, tiles);
+        prefill_kernel<128, true><<<grid, dim3(PP::THREADS), 0, s>>>(a);
+        prefill_merge_kernel<128><<<mgrid, dim3(kMergeThreads), 0, s>>>(a);
       } else {
-        prefill_convert256_kernel<<<dim3(npages), dim3(256), 0, s>>>(a, tiles, h);
-        prefill_tiles256_kernel<<<dim3(static_cast<unsigned>(a.grid)), dim3(PW256::THREADS), 0, s>>>(a);
-        prefill_merge_kernel<256><<<dim3(static_cast<unsigned>(pl.nbh * kMergeSplit)), dim3(kMergeThreads), 0, s>>>(a);
+        prefill_convert256_kernel<<<cgrid, dim3(256), 0, s>>>(a, tiles);
+        prefill_tiles256_kernel<<<grid, dim3(PW256::THREADS), 0, s>>>(a);
+        prefill_merge_kernel<256><<<mgrid, dim3(kMergeThreads), 0, s>>>(a);
       }
       const int rc = launch_status("k8v4_prefill_paged");
       if (rc) return rc;

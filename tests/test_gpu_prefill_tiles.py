@@ -89,3 +89,35 @@ def test_running_max_moves_late_and_often(gpu_ops, d, q_len, seq_len, vmax):
     want = _want(cache, q, table[0], seq_len)
     assert np.abs(want).max() > 0.05 * vmax
     assert_close(_run(cache, q, table[0], seq_len), want, atol=0.022 * vmax, rtol=1e-2, what="rising scores")
+
+
+def test_a_workspace_for_one_head_still_serves_the_call(gpu_ops):
+    """The images of one KV head at a time fit a workspace of the partial
+    states of a one-head launch plus one head's images; a larger one lets
+    several heads share a launch.  Both give the oracle's rows."""
+    lay = PageLayout(4, 128)
+    q_len = seq_len = 1025
+    gen = torch.Generator().manual_seed(1025)
+    pages = -(-seq_len // PAGE)
+    cache = Cache(pages + 3, lay)
+    table = random_tables(gen, [seq_len], pages + 3)
+    fill_sequence(gpu_ops, cache, gen, table[0], seq_len)
+    q = seeded_normal(gen, (q_len, lay.hq, 128))
+    want = _want(cache, q, table[0], seq_len)
+    blocks = -(-q_len * 6 // 256)
+    steps = sum(min(q_len - 1, (256 * b + 255) // 6) // PAGE + 1 for b in range(blocks))
+    grid = min(256, steps // 4) // 8 * 8
+    one_head = (grid * 2 * 256 * 130 * 4 + 255) // 256 * 256 + pages * 35 * 1024
+    full = gpu_ops.prefill_workspace_bytes(seq_len, q_len, 4, 128)
+    assert full > one_head
+    row = table[0].to(device=DEV, dtype=torch.int32)
+    for nbytes in (one_head, full):
+        ws = torch.empty(nbytes // 4, dtype=torch.float32, device=DEV)
+        out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=DEV)
+        gpu_ops.prefill_paged(q.to(DEV), *cache.region_args(), row, seq_len, 1, 1.0 / math.sqrt(128), out, ws)
+        torch.cuda.synchronize()
+        assert_close(out.cpu().numpy(), want, what="%d bytes" % nbytes)
+    with pytest.raises(RuntimeError, match="prefill workspace holds"):
+        gpu_ops.prefill_paged(q.to(DEV), *cache.region_args(), row, seq_len, 1, 1.0 / math.sqrt(128),
+                              torch.empty(q.shape, dtype=torch.float32, device=DEV),
+                              torch.empty(one_head // 4 - 64, dtype=torch.float32, device=DEV))
