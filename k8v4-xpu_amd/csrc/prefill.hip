@@ -1691,10 +1691,326 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
   }
 }
 
+// ---- D = 128 over tile images: four waves of 64 rows, products and vector work
+// interleaved inside each wave ----
+// What bounds it: the power limit.  A large fp16 matrix product reaches 1,318
+// TFLOP/s on this card, far below the 2,500 of its peak clock, and so does any
+// schedule of this attention; what counts is the work per product besides it:
+// tile bytes moved, LDS reads, rescales.  A wave of 64 rows reads each operand
+// from LDS for two MFMAs (a 32-row wave: one), the page order keeps the tile
+// reads in L2 (7.0 -> 0.9 GB a head from beyond it), and a running max that may
+// lag by 2^8 rescales the 128 accumulators rarely (a lag of 2^2 cost 8 %).
+// Measured, 4,224 query tokens over 135,296 keys, 4 KV heads, against two
+// groups of four 32-row waves in ping-pong: 6,080 -> 5,790 us (1,137 -> 1,194
+// TFLOP/s).
+//
+// With no second wave on the SIMD to overlap with, the wave's own instruction
+// stream carries three pages at once, one MFMA per slot with the vector work
+// that fits under it.  Iteration i:
+//   slots  0-31: PV(i - 1)       slots 32-63: QK(i + 1) into the other score buffer
+//   slots  0-7:  row maxima of S(i), then (rarely) the mask and a new running max
+//   slots  8-63: P(i) = exp2(S(i)), written over P(i - 1) behind its last use
+// Score buffers alternate, so the loop is unrolled by two.  A moved running max
+// rescales O at the end of the iteration, when PV(i - 1) -- still relative to
+// the old max -- is in it.
+//
+// Tile q lives in ring slot q % 4.  Iteration i issues K of tile i + 3 and V
+// of tile i + 2 (group G(i): nine 1 KB pieces per wave); its closing wait
+// leaves only G(i) in flight, so iteration i + 1 may read K(i + 2) and
+// V(i + 1).  Slot (i + 3) % 4 held K(i - 1), last read in iteration i - 2, and
+// slot (i + 2) % 4 held V(i - 2), last read in iteration i - 1.
+struct PW128 {
+  static constexpr int D = 128;
+  static constexpr int NW = 4, THREADS = 256, ROWS = 256;
+  static constexpr int SLOTS = 4;
+  static constexpr int PIECES = 9;  // per wave and group: 35 pieces, one of them moved twice
+  static constexpr int LDS = SLOTS * PP::BUF;
+  static_assert(PP::V_OFF == 17 * 1024 && PP::BUF == 35 * 1024, "piece assignment of the DMAs");
+  static_assert(ROWS == Tile<128>::ROWS, "one block shape per head dim");
+};
+
+__device__ __forceinline__ void run_segment_wide(const PrefillArgs &a, char *smem, int h, int rb, int p_lo, int p_hi,
+                                                 PageOrder ord, float *part, int wv, int lane) {
+  constexpr int D = PW128::D, DS = D / 16, DT = D / 32;
+  const int n = p_hi - p_lo;
+  const int nrows = a.q_len * 6;
+  const int row0 = rb * PW128::ROWS;
+  const int hh = lane / 32, r32 = lane % 32;
+
+  // DMAs of group G(j), in five steps: K pieces 4 wv .. + 3 of tile j + 3, V
+  // pieces 4 wv .. + 3 of tile j + 2, then K 16 (waves 0 and 3) or V 16, 17
+  // (waves 1, 2).
+  const char *tiles = a.tiles + (h - a.head0) * a.tile_head;
+  const uint32_t lane16 = 16 * lane;
+  const bool last_v = wv == 1 || wv == 2;
+  const int last_off = last_v ? PP::V_OFF + 1024 * (15 + wv) : 1024 * 16;
+  auto dma_step = [&](int j, int x) {
+    const int q = x < 2 || (x == 4 && !last_v) ? j + 3 : j + 2;
+    const char *src = tiles + static_cast<int64_t>(ord.page(min(max(q, 0), n - 1))) * PP::BUF;
+    lds_t *dst = (lds_t *)(smem + (q & 3) * PP::BUF);
+    const int off = x < 2 ? 4096 * wv + 2048 * x : x < 4 ? PP::V_OFF + 4096 * wv + 2048 * (x - 2) : last_off;
+    if (x < 4)
+      dma_piece_pair(src + off, lane16, dst + off);
+    else
+      dma_piece(src + off, lane16, dst + off);
+  };
+#pragma unroll
+  for (int j = -3; j < 0; ++j)
+#pragma unroll
+    for (int x = 0; x < 5; ++x) dma_step(j, x);
+
+  // ---- query fragments of the two row tiles (B operand of S^T = K Q^T) and
+  // the row limits, as run_segment.
+  v8h qf[2][DS];
+  int lim[2];
+  bool row_valid[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const int row = row0 + wv * 64 + rt * 32 + r32;
+    row_valid[rt] = row < nrows;
+    const int tok = row_valid[rt] ? row / 6 : 0;
+    const int qh = h * 6 + (row_valid[rt] ? row % 6 : 0);
+    lim[rt] = row_valid[rt] ? a.seq_len - a.q_len + tok + 1 : 1;
+    const uint16_t *src = a.q + static_cast<int64_t>(tok) * a.q_tok_stride + static_cast<int64_t>(qh) * D + 8 * hh;
+    if (a.q_bf16) {
+#pragma unroll
+      for (int ds = 0; ds < DS; ++ds) {
+        const uint4 raw = row_valid[rt] ? *reinterpret_cast<const uint4 *>(src + 16 * ds) : make_uint4(0, 0, 0, 0);
+        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          qf[rt][ds][2 * e] = static_cast<_Float16>(__uint_as_float(w[e] << 16));
+          qf[rt][ds][2 * e + 1] = static_cast<_Float16>(__uint_as_float(w[e] & 0xFFFF0000u));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int ds = 0; ds < DS; ++ds) {
+        const uint4 raw = row_valid[rt] ? *reinterpret_cast<const uint4 *>(src + 16 * ds) : make_uint4(0, 0, 0, 0);
+        qf[rt][ds] = __builtin_bit_cast(v8h, raw);
+      }
+    }
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+a"(qf[rt][ds]));
+  }
+  const int tok_lo = row0 / 6;
+  const int full_pages = (a.seq_len - a.q_len + tok_lo + 1) / 64;
+
+  v16f O[2][DT];
+  uint32_t P[2][16];  // packed fp16 pairs, 16-key step st in words 4 st .. + 3
+  v16f sA[2][2], sB[2][2];
+  v16f minit[2];  // -m of the row (0 before its first visible key), the QK accumulators' start
+  float m_run[2], thr[2], lsum[2], alpha_o[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      O[rt][dt] = (v16f)0.f;
+      asm volatile("" : "+a"(O[rt][dt]));
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) P[rt][e] = 0;
+    minit[rt] = (v16f)0.f;
+    m_run[rt] = thr[rt] = -INFINITY;
+    lsum[rt] = 0.f;
+    alpha_o[rt] = 1.f;
+  }
+  auto p_frag = [&](int rt, int st) -> v8h {
+    return __builtin_bit_cast(v8h, make_uint4(P[rt][4 * st], P[rt][4 * st + 1], P[rt][4 * st + 2], P[rt][4 * st + 3]));
+  };
+
+  // Operand reads: fragment f of an iteration feeds the MFMAs of slots 2f and
+  // 2f + 1 (row tiles 0 and 1): V^T (st, dt) = (f / 4, f % 4) of page i - 1
+  // for f < 16, K (kt, ds) = ((f - 16) / 8, f % 8) of page i + 1 after.  They
+  // run AHEAD fragments in front of the products, across the barrier.
+  const char *kbase = smem + r32 * PP::KROW + 16 * hh;
+  const char *vbase = smem + PP::V_OFF + r32 * PP::VROW + 16 * hh;
+  auto k_frag = [&](int q, int f) -> v8h {
+    return *reinterpret_cast<const v8h *>(kbase + (q & 3) * PP::BUF + 32 * (f >> 3) * PP::KROW + 32 * (f & 7));
+  };
+  auto v_frag = [&](int q, int f) -> v8h {
+    return *reinterpret_cast<const v8h *>(vbase + (q & 3) * PP::BUF + 32 * (f & 3) * PP::VROW + 32 * (f >> 2));
+  };
+  constexpr int AHEAD = 8;
+  v8h fr[AHEAD];
+
+  // ---- prologue: S(0) from K(0), then the first operands of V(-1)
+  asm volatile("s_waitcnt vmcnt(18)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int f = 0; f < 16; ++f) {
+    const v8h kf = k_frag(0, f);
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+      if (f & 7)
+        mfma_score(sA[rt][f >> 3], kf, qf[rt][f & 7]);
+      else
+        mfma_score0(sA[rt][f >> 3], kf, qf[rt][f & 7], minit[rt]);
+  }
+#pragma unroll
+  for (int f = 0; f < AHEAD; ++f) fr[f] = v_frag(-1, f);
+  mfma_settle();
+  asm volatile("s_waitcnt vmcnt(9)\n\ts_barrier" ::: "memory");
+
+  // Iteration i: P = P(i - 1) -> P(i), O += V(i - 1) P(i - 1), sc = S(i), sn = S(i + 1).
+  auto iteration = [&](int i, v16f (&sc)[2][2], v16f (&sn)[2][2]) {
+    auto product = [&](auto sl) {
+      constexpr int s = decltype(sl)::value;
+      constexpr int f = s >> 1, rt = s & 1;
+      if constexpr (f < 16)
+        mfma_out(O[rt][f & 3], fr[f % AHEAD], p_frag(rt, f >> 2));
+      else if constexpr (f & 7)
+        mfma_score(sn[rt][(f - 16) >> 3], fr[f % AHEAD], qf[rt][f & 7]);
+      else
+        mfma_score0(sn[rt][(f - 16) >> 3], fr[f % AHEAD], qf[rt][f & 7], minit[rt]);
+      if constexpr (rt == 1) {
+        constexpr int g = f + AHEAD;
+        fr[f % AHEAD] = g < 16 ? v_frag(i - 1, g) : g < 32 ? k_frag(i + 1, g - 16) : v_frag(i, g - 32);
+      }
+    };
+    float mx[2] = {-INFINITY, -INFINITY};
+    static_for<8>([&](auto sl) {
+      constexpr int s = decltype(sl)::value;
+      product(sl);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int r = k & 1, e = 4 * (s & 3) + (k & 2);
+        mx[r] = fmaxf(fmaxf(mx[r], sc[r][s >> 2][e]), sc[r][s >> 2][e + 1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    const int p = ord.page(i);
+    if (__builtin_expect(p >= full_pages, 0)) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        mx[rt] = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            if (p * 64 + 32 * kt + 8 * (e >> 2) + 4 * hh + (e & 3) >= lim[rt]) sc[rt][kt][e] = -INFINITY;
+            mx[rt] = fmaxf(mx[rt], sc[rt][kt][e]);
+          }
+      }
+    }
+    // A row's max passes the threshold exactly when one of its two lanes'
+    // does, so the cross-lane max is only taken on a rescale.
+    const bool moved = __ballot(mx[0] > thr[0] || mx[1] > thr[1]) != 0;
+    if (moved) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        const float m_use = m_run[rt] == -INFINITY ? 0.f : m_run[rt];
+        auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx[rt]), __float_as_uint(mx[rt]), false, false);
+        const float rmx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) + m_use;
+        const float mnew = fmaxf(m_run[rt], rmx);
+        alpha_o[rt] = m_run[rt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[rt] - mnew);
+        m_run[rt] = mnew;
+        lsum[rt] *= alpha_o[rt];
+        const float m_new_use = mnew == -INFINITY ? 0.f : mnew;
+        minit[rt] = (v16f)(-m_new_use);
+        thr[rt] = mnew == -INFINITY ? -INFINITY : 8.f;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) sc[rt][kt] -= m_new_use - m_use;
+      }
+    }
+    float pr0 = 0.f;
+    static_for<56>([&](auto sl) {
+      constexpr int s = 8 + decltype(sl)::value;
+      product(std::integral_constant<int, s>{});
+      // P(i), 8 scores over every 7 slots: score x is key step st, row tile r.
+      constexpr int x0 = (s - 8) * 8 / 7, x1 = (s - 7) * 8 / 7;
+#pragma unroll
+      for (int x = x0; x < x1; ++x) {
+        const int st = x >> 4, r = (x >> 3) & 1, j = x & 7;
+        const float pr = __builtin_amdgcn_exp2f(sc[r][st >> 1][8 * (st & 1) + j]);
+        lsum[r] += pr;
+        asm volatile("" : "+v"(lsum[r]));
+        if (j & 1) {
+          const v2h two = {static_cast<_Float16>(pr0), static_cast<_Float16>(pr)};
+          P[r][4 * st + (j >> 1)] = __builtin_bit_cast(uint32_t, two);
+          asm volatile("" : "+v"(P[r][4 * st + (j >> 1)]));  // computed here, not where it is used
+        } else {
+          pr0 = pr;
+        }
+      }
+      if constexpr (s % 11 == 9) dma_step(i, s / 11);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if (__builtin_expect(moved && i > 0, 0)) {  // at i = 0 O is zero
+      mfma_settle();
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc_scale(O[rt][dt], e, alpha_o[rt]);
+        }
+    }
+    // All but this iteration's pieces have landed, for every wave after the barrier.
+    asm volatile("s_waitcnt vmcnt(9)\n\ts_barrier" ::: "memory");
+  };
+  for (int i = 0; i < n; i += 2) {
+    iteration(i, sA, sB);
+    if (i + 1 >= n) break;
+    iteration(i + 1, sB, sA);
+  }
+  mfma_settle();
+#pragma unroll
+  for (int f = 0; f < 16; ++f) {
+    const v8h vf = f < AHEAD ? fr[f] : v_frag(n - 1, f);
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) mfma_out(O[rt][f & 3], vf, p_frag(rt, f >> 2));
+  }
+  // Nothing in flight when the ring is reused or the work-group ends.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_barrier();
+  mfma_settle();
+
+  // ---- finalize: O = 16 acc / l (V^T holds V / 16)
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum[rt]), __float_as_uint(lsum[rt]), false, false);
+    const float l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    if (part) {
+      const int lr = wv * 64 + rt * 32 + r32;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v4f o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = 16.f * O[rt][dt][4 * j + e];
+          *reinterpret_cast<v4f *>(part + lr * D + 32 * dt + 8 * j + 4 * hh) = o;
+        }
+      if (hh == 0) {
+        part[PW128::ROWS * D + lr] = m_run[rt];
+        part[PW128::ROWS * D + PW128::ROWS + lr] = l;
+      }
+    } else if (row_valid[rt]) {
+      const int row = row0 + wv * 64 + rt * 32 + r32;
+      const float inv = l > 0.f ? 16.f / l : 0.f;
+      const int tok = row / 6, qh = h * 6 + row % 6;
+      const int64_t ob = static_cast<int64_t>(tok) * a.out_tok_stride + static_cast<int64_t>(qh) * D + 4 * hh;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v4f o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = O[rt][dt][4 * j + e] * inv;
+          store_out4(a.out, a.out_dtype, ob + 32 * dt + 8 * j, o);
+        }
+    }
+  }
+}
+
 // Attention of KV heads over their tile images.
-__global__ __attribute__((amdgpu_flat_work_group_size(PW256::THREADS, PW256::THREADS), amdgpu_waves_per_eu(1, 1))) void
-prefill_tiles256_kernel(PrefillArgs a) {
-  __shared__ __attribute__((aligned(16))) char smem[PW256::LDS];
+template <int D>
+using Wide = std::conditional_t<D == 128, PW128, PW256>;
+template <int D>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1))) void
+prefill_tiles_kernel(PrefillArgs a) {
+  using W = Wide<D>;
+  __shared__ __attribute__((aligned(16))) char smem[W::LDS];
   const int w = blockIdx.x;
   const int v = a.xcd_perm ? (w % 8) * (a.grid / 8) + w / 8 : w;
   const int s0 = range_start(a, v), s1 = range_start(a, v + 1);
@@ -1704,8 +2020,11 @@ prefill_tiles256_kernel(PrefillArgs a) {
   for (int e = s1; e > s0;) {
     const TileSegment g = last_segment(a, s0, s1, e, lane);
     float *part = nullptr;
-    if (!g.whole) part = a.ws + (static_cast<int64_t>(v) * 2 + g.slot) * PW256::ROWS * (PW256::D + 2);
-    run_segment_pair(a, smem, a.head0 + g.hl, g.rb, g.p_lo, g.p_hi, g.order, part, wave, lane);
+    if (!g.whole) part = a.ws + (static_cast<int64_t>(v) * 2 + g.slot) * W::ROWS * (W::D + 2);
+    if constexpr (D == 128)
+      run_segment_wide(a, smem, a.head0 + g.hl, g.rb, g.p_lo, g.p_hi, g.order, part, wave, lane);
+    else
+      run_segment_pair(a, smem, a.head0 + g.hl, g.rb, g.p_lo, g.p_hi, g.order, part, wave, lane);
     e -= g.p_hi - g.p_lo;
   }
 }
@@ -2076,6 +2395,15 @@ int heads_per_launch(int64_t npages, int hkv, int head_dim) {
   return static_cast<int>((hkv + launches - 1) / launches);  // 2 + 2 rather than 3 + 1
 }
 
+// Head dim 128: 64-row waves (prefill_tiles_kernel) from this many pages per
+// segment on, where a segment is a row block or a work-group's share of one;
+// below it their longer ramp (half a page more than the ping-pong groups')
+// outweighs what they save.  4 heads, ping-pong against 64-row waves: 12 pages
+// 68.2 / 72.8 us, 32 pages 304.8 / 311.9, 34 pages (whole prompt of 4,224
+// tokens) 246 / 273, 49 pages 149.3 / 144.2, 157 pages 355 / 347, 805 pages
+// 6,080 / 5,790.
+constexpr int kWideMinPages = 40;
+
 // Host mirror of the device schedule; false if the call is too large for it.
 bool plan_prefill(int64_t seq_len, int64_t q_len, int hkv, int head_dim, PrefillPlan &pl) {
   const int64_t R = rows_per_block(head_dim);
@@ -2277,11 +2605,14 @@ extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stri
       const dim3 mgrid(static_cast<unsigned>(pl.nbh * heads * kMergeSplit));
       if (head_dim == 128) {
         prefill_convert_kernel<<<cgrid, dim3(256), 0, s>>>(a, tiles);
-        prefill_kernel<128, true><<<grid, dim3(PP::THREADS), 0, s>>>(a);
+        if (std::min(a.total / a.grid, pl.tper / pl.nbh) >= kWideMinPages)
+          prefill_tiles_kernel<128><<<grid, dim3(PW128::THREADS), 0, s>>>(a);
+        else
+          prefill_kernel<128, true><<<grid, dim3(PP::THREADS), 0, s>>>(a);
         prefill_merge_kernel<128><<<mgrid, dim3(kMergeThreads), 0, s>>>(a);
       } else {
         prefill_convert256_kernel<<<cgrid, dim3(256), 0, s>>>(a, tiles);
-        prefill_tiles256_kernel<<<grid, dim3(PW256::THREADS), 0, s>>>(a);
+        prefill_tiles_kernel<256><<<grid, dim3(PW256::THREADS), 0, s>>>(a);
         prefill_merge_kernel<256><<<mgrid, dim3(kMergeThreads), 0, s>>>(a);
       }
       const int rc = launch_status("k8v4_prefill_paged");

@@ -43,6 +43,8 @@ def _want(cache, q, row, seq_len):
     # one key in the last page, six rows in the last block
     (2, 256, 2049, 16385),
     (4, 128, 129, 129), (2, 128, 171, 65), (4, 128, 683, 1985), (2, 128, 1999, 1999),
+    # 64-row waves of 128 dims: 40 pages a segment or more
+    (4, 128, 1025, 12801), (2, 128, 2100, 14913), (2, 128, 5000, 6000),
 ])
 def test_segments_of_every_length(gpu_ops, hkv, d, q_len, seq_len):
     seq_len = max(q_len, seq_len)
@@ -59,7 +61,7 @@ def test_segments_of_every_length(gpu_ops, hkv, d, q_len, seq_len):
 
 
 @pytest.mark.parametrize("vmax", [65504.0, 1.0])
-@pytest.mark.parametrize("d,q_len,seq_len", [(256, 2100, 8192), (128, 200, 8192)])
+@pytest.mark.parametrize("d,q_len,seq_len", [(256, 2100, 8192), (128, 200, 8192), (128, 2100, 8192)])
 def test_running_max_moves_late_and_often(gpu_ops, d, q_len, seq_len, vmax):
     """Each 32-token chunk scores 0.25 (log2 units) above the one before, with
     V rows of +-vmax whose sign alternates from chunk to chunk: with the widest
