@@ -82,8 +82,9 @@ struct PrefillArgs {
   float c;       // softmax scale * log2(e)
   int rows;      // query rows per block (32 per wave of a work-group)
   int nbh;       // row blocks per KV head
-  int tper;      // page steps of one head: sum over its blocks of the pages each reads
-  int total;     // page steps of the call (hkv * tper)
+  int tper;      // steps of one head: sum over its blocks of cost + the pages each reads
+  int cost;      // steps without pages at the start of a block
+  int total;     // steps of the launch (its heads * tper)
   int grid;      // persistent work-groups; work-group v takes steps [v*total/grid, (v+1)*total/grid)
   int xcd_perm;  // map ids so the work-groups of one XCD take adjacent work (grid % 8 == 0)
   float *ws;     // partial states: [grid][2][rows][D + 2] floats
@@ -291,17 +292,25 @@ __device__ __forceinline__ void store_out4(void *out, int dtype, int64_t idx, v4
 }
 
 // ---- balanced schedule (shared by the attention and merge kernels)
-// The work of KV head h, row block rb is `block_pages(rb)` page steps; the
-// blocks are laid out head-major as one line of `total` steps, and the
-// persistent work-group v takes steps [v*total/grid, (v+1)*total/grid).  A
-// block split between work-groups is finished by the merge kernel from the
-// partial states the pieces leave in the workspace: the piece of work-group v
-// goes to slot 0 if v's range starts inside the block, else to slot 1.
+// The work of KV head h, row block rb is `block_pages(rb)` page steps behind
+// a.cost steps without pages; the blocks are laid out head-major as one
+// line of `total` steps, and the persistent work-group v takes steps
+// [v*total/grid, (v+1)*total/grid).  A block split between work-groups is
+// finished by the merge kernel from the partial states the pieces leave in the
+// workspace: the piece of work-group v goes to slot 0 if v's range starts
+// inside the block, else to slot 1.
+//
+// The steps without pages stand for what a block costs besides its pages (its
+// query rows, the first tile's latency, the pipeline's ramp, its output): with
+// pages alone counted, a work-group that drew eight one-page blocks took
+// several times as long as one with eight pages of one block (block_cost()).
 
 __device__ __forceinline__ int block_pages(const PrefillArgs &a, int rb) {
   const int tok_hi = min(a.q_len - 1, (rb * a.rows + a.rows - 1) / 6);
   return (a.seq_len - a.q_len + tok_hi + 1 + 63) / 64;
 }
+
+__device__ __forceinline__ int block_steps(const PrefillArgs &a, int rb) { return a.cost + block_pages(a, rb); }
 
 // Block of one head that contains step sp (0 <= sp < tper), and the steps of
 // the blocks before it.  Wave-uniform.
@@ -311,7 +320,7 @@ __device__ __forceinline__ void locate_block(const PrefillArgs &a, int sp, int l
   before = 0;
   for (int r0 = 0; r0 < a.nbh; r0 += 64) {
     const int r = r0 + lane;
-    const int n = r < a.nbh ? block_pages(a, r) : 0;
+    const int n = r < a.nbh ? block_steps(a, r) : 0;
     int incl = n;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -522,6 +531,7 @@ __device__ __forceinline__ void run_segment(const PrefillArgs &a, char *smem, in
     auto a2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(cz), __float_as_uint(cz), false, false);
     cz = __uint_as_float(a2[0]) + __uint_as_float(a2[1]);
   }
+  if (!row_valid) return;  // padding rows: the merge does not read them
   if (part) {
     // Partial segment: O' = acc * 2^24|2^20 - corr (before the division), m, l.
     const int lr = wave * 32 + r32;
@@ -540,7 +550,6 @@ __device__ __forceinline__ void run_segment(const PrefillArgs &a, char *smem, in
     }
     return;
   }
-  if (!row_valid) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
   const int tok = row / 6, qh = h * 6 + row % 6;
   const int64_t ob = static_cast<int64_t>(tok) * a.out_tok_stride + static_cast<int64_t>(qh) * D + 4 * hh;
@@ -1094,6 +1103,7 @@ __device__ __forceinline__ void run_segment_pp(const PrefillArgs &a, char *smem,
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(Lacc[0]), __float_as_uint(Lacc[0]), false, false);
     l = hh == 0 ? Lacc[0] : __uint_as_float(sw[0]);
   }
+  if (!row_valid) return;  // padding rows: the merge does not read them
   if (part) {
     const int lr = wave * 32 + r32;
 #pragma unroll
@@ -1111,7 +1121,6 @@ __device__ __forceinline__ void run_segment_pp(const PrefillArgs &a, char *smem,
     }
     return;
   }
-  if (!row_valid) return;
   const float inv = l > 0.f ? 16.f / l : 0.f;
   const int tok = row / 6, qh = h * 6 + row % 6;
   const int64_t ob = static_cast<int64_t>(tok) * a.out_tok_stride + static_cast<int64_t>(qh) * D + 4 * hh;
@@ -1143,26 +1152,27 @@ struct PageOrder {
     return p < p_hi ? p : p - (p_hi - p_lo);
   }
 };
-struct TileSegment {
-  int hl, rb, p_lo, p_hi, slot;
-  bool whole;
+struct Segment {
+  int hl, rb, p_lo, p_hi;  // pages [p_lo, p_hi) of a row block (none if p_lo == p_hi)
+  int begin;               // first step of the segment
+  int slot;                // partial state's slot, or -1 for a whole block
   PageOrder order;
 };
 
 // The last segment of the steps [s0, e) of a work-group that owns [s0, s1).
-__device__ __forceinline__ TileSegment last_segment(const PrefillArgs &a, int s0, int s1, int e, int lane) {
-  TileSegment g;
+__device__ __forceinline__ Segment last_segment(const PrefillArgs &a, int s0, int s1, int e, int lane) {
+  Segment g;
   g.hl = (e - 1) / a.tper;
   int before;
   locate_block(a, e - 1 - g.hl * a.tper, lane, g.rb, before);
   const int base = g.hl * a.tper + before;
   const int n = block_pages(a, g.rb);
-  g.p_lo = max(0, s0 - base);
-  g.p_hi = e - base;
-  g.slot = s0 >= base ? 0 : 1;
-  g.whole = g.p_lo == 0 && g.p_hi == n;
+  g.begin = max(s0, base);
+  g.p_lo = max(0, g.begin - base - a.cost);
+  g.p_hi = max(0, e - base - a.cost);
+  g.slot = g.p_lo == 0 && g.p_hi == n ? -1 : s0 >= base ? 0 : 1;
   int start = g.p_lo;
-  if (g.whole) {
+  if (g.slot < 0) {
     start = (s1 - e) % n;
   } else if (s0 >= base && e == s1) {
     const int T = a.total / a.grid + 1;
@@ -1658,6 +1668,7 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt) {
     const int row = row0 + rt * 32 + r32;
+    if (!row_valid[rt]) continue;  // padding rows: the merge does not read them
     if (part) {
       const int lr = row - rb * PW256::ROWS;
 #pragma unroll
@@ -1673,7 +1684,7 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
         part[PW256::ROWS * D + lr] = m_run[rt];
         part[PW256::ROWS * D + PW256::ROWS + lr] = l[rt];
       }
-    } else if (row_valid[rt]) {
+    } else {
       const float inv = l[rt] > 0.f ? 1.f / l[rt] : 0.f;
       const int tok = row / 6, qh = h * 6 + row % 6;
       const int64_t ob =
@@ -1970,6 +1981,7 @@ __device__ __forceinline__ void run_segment_wide(const PrefillArgs &a, char *sme
   for (int rt = 0; rt < 2; ++rt) {
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum[rt]), __float_as_uint(lsum[rt]), false, false);
     const float l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    if (!row_valid[rt]) continue;  // padding rows: the merge does not read them
     if (part) {
       const int lr = wv * 64 + rt * 32 + r32;
 #pragma unroll
@@ -1985,7 +1997,7 @@ __device__ __forceinline__ void run_segment_wide(const PrefillArgs &a, char *sme
         part[PW128::ROWS * D + lr] = m_run[rt];
         part[PW128::ROWS * D + PW128::ROWS + lr] = l;
       }
-    } else if (row_valid[rt]) {
+    } else {
       const int row = row0 + wv * 64 + rt * 32 + r32;
       const float inv = l > 0.f ? 16.f / l : 0.f;
       const int tok = row / 6, qh = h * 6 + row % 6;
@@ -2018,14 +2030,15 @@ prefill_tiles_kernel(PrefillArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int lane = threadIdx.x % 64;
   for (int e = s1; e > s0;) {
-    const TileSegment g = last_segment(a, s0, s1, e, lane);
+    const Segment g = last_segment(a, s0, s1, e, lane);
+    e = g.begin;
+    if (g.p_lo == g.p_hi) continue;
     float *part = nullptr;
-    if (!g.whole) part = a.ws + (static_cast<int64_t>(v) * 2 + g.slot) * W::ROWS * (W::D + 2);
+    if (g.slot >= 0) part = a.ws + (static_cast<int64_t>(v) * 2 + g.slot) * W::ROWS * (W::D + 2);
     if constexpr (D == 128)
       run_segment_wide(a, smem, a.head0 + g.hl, g.rb, g.p_lo, g.p_hi, g.order, part, wave, lane);
     else
       run_segment_pair(a, smem, a.head0 + g.hl, g.rb, g.p_lo, g.p_hi, g.order, part, wave, lane);
-    e -= g.p_hi - g.p_lo;
   }
 }
 
@@ -2048,25 +2061,23 @@ prefill_kernel(PrefillArgs a) {
     // The ping-pong ring starts zeroed: its tiles then only ever hold finite values.
     for (int o = 16 * tid; o < 4 * PP::BUF; o += 16 * PP::THREADS) *reinterpret_cast<uint4 *>(smem + o) = make_uint4(0, 0, 0, 0);
   }
-  int s = s0;
-  bool first = true;
-  while (s < s1) {
+  for (int s = s0; s < s1;) {
     const int hl = s / a.tper;
-    const int h = a.head0 + hl;
     int rb, before;
     locate_block(a, s - hl * a.tper, lane, rb, before);
+    const int base = hl * a.tper + before;
     const int n = block_pages(a, rb);
-    const int p_lo = s - hl * a.tper - before;
-    const int p_hi = min(n, p_lo + (s1 - s));
+    const int end = min(s1, base + a.cost + n);
+    const int p_lo = max(0, s - base - a.cost), p_hi = max(0, end - base - a.cost);
+    s = end;
+    if (p_lo == p_hi) continue;
     float *part = nullptr;
     if (p_lo != 0 || p_hi != n)
-      part = a.ws + (static_cast<int64_t>(v) * 2 + (first ? 0 : 1)) * T::ROWS * (D + 2);
+      part = a.ws + (static_cast<int64_t>(v) * 2 + (s0 >= base ? 0 : 1)) * T::ROWS * (D + 2);
     if constexpr (D == 128)
-      run_segment_pp<PRE>(a, smem, h, rb, p_lo, p_hi, part, tid, wave, lane);
+      run_segment_pp<PRE>(a, smem, a.head0 + hl, rb, p_lo, p_hi, part, tid, wave, lane);
     else
-      run_segment<D>(a, smem, h, rb, p_lo, p_hi, part, tid, wave, lane);
-    s += p_hi - p_lo;
-    first = false;
+      run_segment<D>(a, smem, a.head0 + hl, rb, p_lo, p_hi, part, tid, wave, lane);
   }
 }
 
@@ -2161,7 +2172,7 @@ __device__ __forceinline__ int steps_before_block(const PrefillArgs &a, int rb, 
   int base = 0;
   for (int r0 = 0; r0 < rb; r0 += 64) {
     const int r = r0 + lane;
-    base += wave_sum(r < rb ? block_pages(a, r) : 0);
+    base += wave_sum(r < rb ? block_steps(a, r) : 0);
   }
   return base;
 }
@@ -2175,7 +2186,7 @@ __device__ __forceinline__ void merge_block(const PrefillArgs &a, const PrefillA
   constexpr int R = Tile<D>::ROWS, TPR = kMergeTPR<D>, DT = D / TPR;  // DT = 32 dims per thread
   static_assert(DT == 32, "32 dims per merge thread");
   const int n = block_pages(sa, rb);
-  const int va = range_owner(a, start), vb = range_owner(a, start + n - 1);
+  const int va = range_owner(a, start + sa.cost), vb = range_owner(a, start + sa.cost + n - 1);
   if (va == vb) return;  // one work-group did the whole block
   const int lr = part * (R / kMergeSplit) + threadIdx.x / TPR, sub = threadIdx.x % TPR;
   const int row = rb * R + lr;
@@ -2300,26 +2311,26 @@ prefill_batch_kernel(PrefillBatchArgs ba) {
   if constexpr (D == 128) {
     for (int o = 16 * tid; o < 4 * PP::BUF; o += 16 * PP::THREADS) *reinterpret_cast<uint4 *>(smem + o) = make_uint4(0, 0, 0, 0);
   }
-  int s = s0;
-  bool first = true;
-  while (s < s1) {
+  for (int s = s0; s < s1;) {
     const int i = batch_find(ba.step0, ba.n, s);
     const PrefillArgs &sa = batch_seq(i);
-    const int sl = s - batch_off(ba.step0, i);  // step within the sequence
-    const int h = sl / sa.tper;
+    const int first = batch_off(ba.step0, i);  // step line of the sequence
+    const int h = (s - first) / sa.tper;
     int rb, before;
-    locate_block(sa, sl - h * sa.tper, lane, rb, before);
+    locate_block(sa, s - first - h * sa.tper, lane, rb, before);
+    const int base = first + h * sa.tper + before;
     const int n = block_pages(sa, rb);
-    const int p_lo = sl - h * sa.tper - before;
-    const int p_hi = min(n, p_lo + (s1 - s));
+    const int end = min(s1, base + a.cost + n);
+    const int p_lo = max(0, s - base - a.cost), p_hi = max(0, end - base - a.cost);
+    s = end;
+    if (p_lo == p_hi) continue;
     float *part = nullptr;
-    if (p_lo != 0 || p_hi != n) part = a.ws + (static_cast<int64_t>(v) * 2 + (first ? 0 : 1)) * T::ROWS * (D + 2);
+    if (p_lo != 0 || p_hi != n)
+      part = a.ws + (static_cast<int64_t>(v) * 2 + (s0 >= base ? 0 : 1)) * T::ROWS * (D + 2);
     if constexpr (D == 128)
       run_segment_pp<false>(sa, smem, h, rb, p_lo, p_hi, part, tid, wave, lane);
     else
       run_segment<D>(sa, smem, h, rb, p_lo, p_hi, part, tid, wave, lane);
-    s += p_hi - p_lo;
-    first = false;
   }
 }
 
@@ -2341,7 +2352,9 @@ namespace k8v4 {
 namespace {
 
 struct PrefillPlan {
-  int nbh, tper, total, grid;
+  int nbh, tper, total;  // as PrefillArgs, total over all heads
+  int64_t pages;         // pages the blocks of one head read
+  int grid;
   bool tiles;  // pages dequantized once per KV head into tile images
   int heads;   // tiles: KV heads per launch
 };
@@ -2350,6 +2363,13 @@ struct PrefillPlan {
 // 64-token chunk over 2,000 keys: 8 such calls 741 -> 339 us with 4 instead
 // of 1; 8 gave no more).
 constexpr int64_t kMinSteps = 4;
+
+// What a row block costs besides its pages, in page steps.  8 chunks of 17-128
+// tokens over 0.1K-8K (4 heads of 128 dims): 109 us with 0, 82, 70, 64, 63.0,
+// 63.7 us with 1, 2, 3, 4, 6; a whole prompt of 1,999 tokens 100 -> 69 us with
+// 4.  Head dim 256 (a page step takes longer): the same chunks 231 us with 0,
+// 149, 127, 127, 131 us with 1, 2, 3, 4.
+int block_cost(int head_dim) { return head_dim == 128 ? 4 : 2; }
 
 int rows_per_block(int head_dim) { return head_dim == 128 ? Tile<128>::ROWS : Tile<256>::ROWS; }
 
@@ -2370,12 +2390,21 @@ bool tiles_pay_off(int64_t nbh, int64_t npages, int head_dim) {
 
 int64_t tile_stride(int head_dim) { return head_dim == 128 ? PP::BUF : PW256::IMG; }
 
-// Persistent work-groups for a launch of `steps` page steps: one per CU, each
-// with at least kMinSteps steps (a work-group's fixed work -- its query rows,
-// its partial state, the merge's reads of it -- outweighs a page or two of
-// attention), a multiple of 8 from 8 up (whole XCDs).
+// Persistent work-groups for a launch of `steps` steps: one per CU, each with
+// about kMinSteps steps (a work-group's fixed work -- its query rows, its
+// partial state, the merge's reads of it -- outweighs a page or two of
+// attention), whole XCDs (a multiple of 8) from 8 up.  Rounded up, so that no
+// work-group takes a fifth step: 600 steps (50 tokens over 3,000, 4 heads of
+// 256 dims) took 53.2 us as 144 work-groups, 51.8 us as 152.
 int64_t persistent_grid(int64_t steps) {
-  int64_t grid = std::min<int64_t>(static_cast<int64_t>(device_cus()), std::max<int64_t>(1, steps / kMinSteps));
+  const int64_t cus = device_cus();
+  int64_t grid = std::min<int64_t>(cus, std::max<int64_t>(1, (steps + kMinSteps - 1) / kMinSteps));
+  if (grid >= 8) grid = std::min((grid + 7) / 8 * 8, cus / 8 * 8);
+  return grid;
+}
+// The fewest a workspace has to hold: page steps alone, rounded down.
+int64_t least_grid(int64_t pages) {
+  int64_t grid = std::min<int64_t>(static_cast<int64_t>(device_cus()), std::max<int64_t>(1, pages / kMinSteps));
   if (grid >= 8) grid -= grid % 8;
   return grid;
 }
@@ -2408,16 +2437,18 @@ constexpr int kWideMinPages = 40;
 bool plan_prefill(int64_t seq_len, int64_t q_len, int hkv, int head_dim, PrefillPlan &pl) {
   const int64_t R = rows_per_block(head_dim);
   const int64_t nbh = (q_len * kGqa + R - 1) / R;
-  int64_t tper = 0;
+  int64_t pages = 0;
   for (int64_t rb = 0; rb < nbh; ++rb) {
     const int64_t tok_hi = std::min<int64_t>(q_len - 1, (rb * R + R - 1) / 6);
-    tper += (seq_len - q_len + tok_hi + 1 + 63) / 64;
+    pages += (seq_len - q_len + tok_hi + 1 + 63) / 64;
   }
+  const int64_t tper = pages + nbh * block_cost(head_dim);
   const int64_t total = tper * hkv;
   if (nbh < 1 || total < 1 || total >= (int64_t(1) << 31) / 2) return false;
   pl.nbh = static_cast<int>(nbh);
   pl.tper = static_cast<int>(tper);
   pl.total = static_cast<int>(total);
+  pl.pages = pages;
   pl.tiles = tiles_pay_off(nbh, (seq_len + kPage - 1) / kPage, head_dim);
   // The grid of the launch that runs: with tile images over the steps of
   // pl.heads KV heads, else over all heads.
@@ -2445,12 +2476,15 @@ int64_t workspace_size(const PrefillPlan &pl, int64_t seq_len, int hkv, int head
   return (partial_bytes(static_cast<int>(persistent_grid(static_cast<int64_t>(pl.tper) * hkv)), head_dim) + 255) / 256 * 256 +
          pages * tile_stride(head_dim);
 }
-// Fewer heads a launch, down to one, until the call fits `bytes`.
+// A smaller workspace than workspace_size() still serves a call that fits it
+// with fewer heads a launch, down to one, and with the work-groups counted by
+// page steps alone.
 void fit_workspace(PrefillPlan &pl, int64_t seq_len, int head_dim, int64_t bytes) {
   while (pl.tiles && pl.heads > 1 && workspace_need(pl, seq_len, head_dim) > bytes) {
     --pl.heads;
     pl.grid = static_cast<int>(persistent_grid(static_cast<int64_t>(pl.tper) * pl.heads));
   }
+  if (workspace_need(pl, seq_len, head_dim) > bytes) pl.grid = static_cast<int>(least_grid(pl.pages * pl.heads));
 }
 
 // Argument checks shared by the single-sequence and batched prefill entries.
@@ -2581,6 +2615,7 @@ extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stri
   a.rows = rows_per_block(head_dim);
   a.nbh = pl.nbh;
   a.tper = pl.tper;
+  a.cost = block_cost(head_dim);
   a.total = pl.total;
   a.grid = pl.grid;
   a.xcd_perm = pl.grid % 8 == 0 ? 1 : 0;
@@ -2599,13 +2634,13 @@ extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stri
       const int heads = std::min(pl.heads, hkv - h);
       a.head0 = h;
       a.total = pl.tper * heads;
-      a.grid = static_cast<int>(persistent_grid(a.total));
+      a.grid = std::min(pl.grid, static_cast<int>(persistent_grid(a.total)));
       a.xcd_perm = a.grid % 8 == 0 ? 1 : 0;
       const dim3 cgrid(npages, static_cast<unsigned>(heads)), grid(static_cast<unsigned>(a.grid));
       const dim3 mgrid(static_cast<unsigned>(pl.nbh * heads * kMergeSplit));
       if (head_dim == 128) {
         prefill_convert_kernel<<<cgrid, dim3(256), 0, s>>>(a, tiles);
-        if (std::min(a.total / a.grid, pl.tper / pl.nbh) >= kWideMinPages)
+        if (std::min(pl.pages * heads / a.grid, pl.pages / pl.nbh) >= kWideMinPages)
           prefill_tiles_kernel<128><<<grid, dim3(PW128::THREADS), 0, s>>>(a);
         else
           prefill_kernel<128, true><<<grid, dim3(PP::THREADS), 0, s>>>(a);
@@ -2718,6 +2753,7 @@ extern "C" int k8v4_prefill_paged_batch(const void *q, int q_dtype, int64_t q_to
       sa.seq_len = static_cast<int>(seq_lens[i]);
       sa.nbh = pl.nbh;
       sa.tper = pl.tper;
+      sa.cost = block_cost(head_dim);
       ba.step0[k] = static_cast<int>(steps);
       ba.block0[k] = static_cast<int>(blocks);
       steps += pl.total;

@@ -123,3 +123,29 @@ def test_a_workspace_for_one_head_still_serves_the_call(gpu_ops):
         gpu_ops.prefill_paged(q.to(DEV), *cache.region_args(), row, seq_len, 1, 1.0 / math.sqrt(128),
                               torch.empty(q.shape, dtype=torch.float32, device=DEV),
                               torch.empty(one_head // 4 - 64, dtype=torch.float32, device=DEV))
+
+
+@pytest.mark.parametrize("d", [128, 256])
+def test_batch_of_blocks_of_very_different_length(gpu_ops, d):
+    """Row blocks of one page beside blocks of many in one launch: work-groups
+    take many short blocks or a part of a long one, and a work-group's range may
+    begin or end within the steps that stand for a block's fixed cost."""
+    q_lens, ctxs = [11, 64, 128, 17, 33, 90, 12, 100], [0, 0, 9000, 47, 640, 2000, 52, 0]
+    lens = [q + c for q, c in zip(q_lens, ctxs)]
+    lay = PageLayout(2, d)
+    gen = torch.Generator().manual_seed(77 + d)
+    pool = sum(-(-n // PAGE) for n in lens) + 3
+    cache = Cache(pool, lay)
+    table = random_tables(gen, lens, pool)
+    for b, n in enumerate(lens):
+        fill_sequence(gpu_ops, cache, gen, table[b], n)
+    q = seeded_normal(gen, (sum(q_lens), lay.hq, d))
+    out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=DEV)
+    ws = torch.empty(gpu_ops.prefill_batch_workspace_bytes(2, d) // 4, dtype=torch.float32, device=DEV)
+    tok0 = [sum(q_lens[:i]) for i in range(len(q_lens))]
+    gpu_ops.prefill_paged_batch(q.to(DEV), *cache.region_args(), table.to(DEV), tok0, q_lens, lens,
+                                list(range(len(lens))), 1, 1.0 / math.sqrt(d), out, ws)
+    torch.cuda.synchronize()
+    for b, n in enumerate(lens):
+        rows = slice(tok0[b], tok0[b] + q_lens[b])
+        assert_close(out[rows].cpu().numpy(), _want(cache, q[rows], table[b], n), what="sequence %d" % b)
