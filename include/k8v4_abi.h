@@ -198,9 +198,12 @@ int k8v4_attn_batch_profiled(const void *q, int q_dtype, int64_t q_tok_stride,
  * workspace: caller-owned device scratch (16-byte aligned) of workspace_bytes
  *      >= k8v4_prefill_workspace_bytes(seq_len, q_len, hkv, head_dim): partial
  *      softmax states of the row blocks the balanced schedule splits between
- *      work-groups and, for head_dim 128 with q_len * 6 > 768 query rows per
- *      KV head, one head's pages dequantized into MFMA tile images (35,840
- *      bytes per 64-token page; the heads run one after another over it).
+ *      work-groups and, for longer chunks, the pages of one or more KV heads
+ *      dequantized into MFMA tile images (35,840 bytes per 64-token page at
+ *      head_dim 128, 67,584 at 256; as many heads share a launch as fit 128
+ *      MiB).  A workspace with room for one head's images, or at head_dim 256
+ *      where k8v4_prefill_uses_tiles is 0 for the partial states alone, still
+ *      serves the call, more slowly.
  * q_len == 0 is a no-op; q_len > seq_len is an error.
  */
 int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stride, const int8_t *k_cache,
@@ -224,8 +227,9 @@ int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stride, const i
  * take up to 10 non-empty sequences, whose (KV head, row block) work shares
  * the persistent work-groups of one launch; more sequences take more
  * launches, in order, on the stream.  Pages are dequantized in the kernel
- * (no per-head tile pre-pass), which suits short chunks: a long chunk is
- * faster through k8v4_prefill_paged.  The same bottom-right causal rule,
+ * (no per-head tile pre-pass), which suits short chunks; a chunk that
+ * k8v4_prefill_paged would serve from tile images runs that way, by itself,
+ * if the workspace has room for it.  The same bottom-right causal rule,
  * numerics and errors per sequence as k8v4_prefill_paged; q_lens[i] == 0
  * sequences are skipped; nseq == 0 is a no-op.  The library sees neither
  * the table's row count nor the token count of q and out: the caller keeps
@@ -289,10 +293,11 @@ int64_t k8v4_decode_fault_count(void);
  * gathered K/V per head inside the call, onednn_prefill.py:226-239). */
 int64_t k8v4_prefill_workspace_bytes(int64_t seq_len, int64_t q_len, int hkv, int head_dim);
 
-/* Whether k8v4_prefill_paged serves this shape from per-KV-head tile images
- * (each page dequantized once per head; 1), or converts pages in place as
- * k8v4_prefill_paged_batch does (0); -1 on bad arguments.  No counterpart in
- * the reference: a caller batching a step's chunks sends the former alone. */
+/* Whether k8v4_prefill_paged always serves this shape from per-KV-head tile
+ * images (each page dequantized once per head; 1), or may convert pages in
+ * place, as k8v4_prefill_paged_batch does for a step's short chunks together
+ * (0); -1 on bad arguments.  No counterpart in the reference: a caller
+ * batching a step's chunks sends the former alone. */
 int k8v4_prefill_uses_tiles(int64_t seq_len, int64_t q_len, int hkv, int head_dim);
 
 /* Workspace bytes k8v4_attn_batch needs for this shape (-1 on bad arguments).

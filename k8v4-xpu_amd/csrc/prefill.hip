@@ -2356,6 +2356,7 @@ struct PrefillPlan {
   int64_t pages;         // pages the blocks of one head read
   int grid;
   bool tiles;  // pages dequantized once per KV head into tile images
+  bool alone;  // k8v4_prefill_uses_tiles: tile images with any workspace the call takes
   int heads;   // tiles: KV heads per launch
 };
 
@@ -2378,14 +2379,22 @@ int rows_per_block(int head_dim) { return head_dim == 128 ? Tile<128>::ROWS : Ti
 // in-kernel conversion costs less than the extra tile traffic).
 constexpr int kPreMinBlocks = 4;
 
-// Head dim 256 (one wave per SIMD, whose conversion is cheaper in place): per
-// KV head the tile path costs about 59 us of launches and pre-pass latency
-// plus 62 ns per page and saves about 9 ns per (row block, page) -- measured
-// against the in-place conversion over contexts of 4K-64K tokens and chunks
-// of 96-4,224 tokens (two heads; per head either way).
+// Head dim 256: the calls that only ever ran over tile images, whose workspace
+// has to hold them (62 ns per page and 59 us of launches per KV head against
+// 9 ns per row block and page, with the kernels these figures were taken on).
 bool tiles_pay_off(int64_t nbh, int64_t npages, int head_dim) {
   if (nbh < kPreMinBlocks) return false;
   return head_dim == 128 || (9 * nbh - 62) * npages > 58600;
+}
+
+// Head dim 256, other calls of more than 128 tokens, if the workspace has room:
+// the images cost about 10 ns per (page, head) and 19 us a call, and save 10 ns
+// per (row block, page, head).  In place against over images: 512 tokens over
+// 7,777, 4 heads, 243 -> 148 us; 512 over 16,384, 2 heads, 249 -> 149; whole
+// prompt of 2,000, 4 heads, 174 -> 154; of 1,000 (pages - images = 1,516)
+// 75.6 -> 70.5; 512 over 100 (536) 48.7 -> 54.9.
+bool images_pay_off(int64_t nbh, int64_t pages, int64_t npages, int hkv, int head_dim) {
+  return head_dim == 256 && nbh > 6 && (pages - npages) * hkv > 1900;
 }
 
 int64_t tile_stride(int head_dim) { return head_dim == 128 ? PP::BUF : PW256::IMG; }
@@ -2449,7 +2458,8 @@ bool plan_prefill(int64_t seq_len, int64_t q_len, int hkv, int head_dim, Prefill
   pl.tper = static_cast<int>(tper);
   pl.total = static_cast<int>(total);
   pl.pages = pages;
-  pl.tiles = tiles_pay_off(nbh, (seq_len + kPage - 1) / kPage, head_dim);
+  pl.alone = tiles_pay_off(nbh, (seq_len + kPage - 1) / kPage, head_dim);
+  pl.tiles = pl.alone || images_pay_off(nbh, pages, (seq_len + kPage - 1) / kPage, hkv, head_dim);
   // The grid of the launch that runs: with tile images over the steps of
   // pl.heads KV heads, else over all heads.
   pl.heads = pl.tiles ? heads_per_launch((seq_len + kPage - 1) / kPage, hkv, head_dim) : hkv;
@@ -2477,12 +2487,18 @@ int64_t workspace_size(const PrefillPlan &pl, int64_t seq_len, int hkv, int head
          pages * tile_stride(head_dim);
 }
 // A smaller workspace than workspace_size() still serves a call that fits it
-// with fewer heads a launch, down to one, and with the work-groups counted by
-// page steps alone.
+// with fewer heads a launch, down to one, in place where the call is not one
+// that always runs over tile images, and with the work-groups counted by page
+// steps alone.
 void fit_workspace(PrefillPlan &pl, int64_t seq_len, int head_dim, int64_t bytes) {
   while (pl.tiles && pl.heads > 1 && workspace_need(pl, seq_len, head_dim) > bytes) {
     --pl.heads;
     pl.grid = static_cast<int>(persistent_grid(static_cast<int64_t>(pl.tper) * pl.heads));
+  }
+  if (workspace_need(pl, seq_len, head_dim) > bytes && pl.tiles && !pl.alone) {
+    pl.tiles = false;
+    pl.heads = pl.total / pl.tper;  // in place: all heads in one launch
+    pl.grid = static_cast<int>(persistent_grid(pl.total));
   }
   if (workspace_need(pl, seq_len, head_dim) > bytes) pl.grid = static_cast<int>(least_grid(pl.pages * pl.heads));
 }
@@ -2512,6 +2528,40 @@ int check_prefill_args(const void *q, int q_dtype, int64_t q_tok_stride, const i
                    vs_page_stride % 4 == 0 && vz_page_stride % 4 == 0,
                "scale planes must be 4-byte aligned");
   K8V4_REQUIRE(scale > 0.f && scale < 1e30f, "softmax scale must be positive and finite");
+  return K8V4_OK;
+}
+
+// One sequence over tile images, pl.heads KV heads at a time: their pages
+// dequantized once into the workspace, then all row blocks of those heads over
+// them, then their merge.
+int launch_over_tiles(PrefillArgs a, const PrefillPlan &pl, void *workspace, int hkv, int head_dim, hipStream_t s) {
+  char *tiles = static_cast<char *>(workspace) + tiles_offset(pl, head_dim);
+  const unsigned npages = static_cast<unsigned>((a.seq_len + kPage - 1) / kPage);
+  a.tiles = tiles;
+  a.tile_head = static_cast<int64_t>(npages) * tile_stride(head_dim);
+  for (int h = 0; h < hkv; h += pl.heads) {
+    const int heads = std::min(pl.heads, hkv - h);
+    a.head0 = h;
+    a.total = pl.tper * heads;
+    a.grid = std::min(pl.grid, static_cast<int>(persistent_grid(a.total)));
+    a.xcd_perm = a.grid % 8 == 0 ? 1 : 0;
+    const dim3 cgrid(npages, static_cast<unsigned>(heads)), grid(static_cast<unsigned>(a.grid));
+    const dim3 mgrid(static_cast<unsigned>(pl.nbh * heads * kMergeSplit));
+    if (head_dim == 128) {
+      prefill_convert_kernel<<<cgrid, dim3(256), 0, s>>>(a, tiles);
+      if (std::min(pl.pages * heads / a.grid, pl.pages / pl.nbh) >= kWideMinPages)
+        prefill_tiles_kernel<128><<<grid, dim3(PW128::THREADS), 0, s>>>(a);
+      else
+        prefill_kernel<128, true><<<grid, dim3(PP::THREADS), 0, s>>>(a);
+      prefill_merge_kernel<128><<<mgrid, dim3(kMergeThreads), 0, s>>>(a);
+    } else {
+      prefill_convert256_kernel<<<cgrid, dim3(256), 0, s>>>(a, tiles);
+      prefill_tiles_kernel<256><<<grid, dim3(PW256::THREADS), 0, s>>>(a);
+      prefill_merge_kernel<256><<<mgrid, dim3(kMergeThreads), 0, s>>>(a);
+    }
+    const int rc = launch_status("k8v4_prefill_paged");
+    if (rc) return rc;
+  }
   return K8V4_OK;
 }
 
@@ -2564,7 +2614,7 @@ extern "C" int k8v4_prefill_uses_tiles(int64_t seq_len, int64_t q_len, int hkv, 
   if (q_len == 0) return 0;
   PrefillPlan pl;
   if (!plan_prefill(seq_len, q_len, hkv, head_dim, pl)) return -1;
-  return pl.tiles ? 1 : 0;
+  return pl.alone ? 1 : 0;
 }
 
 extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stride, const int8_t *k_cache,
@@ -2623,38 +2673,7 @@ extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stri
   a.head0 = 0;
   a.tiles = nullptr;
   auto s = static_cast<hipStream_t>(stream);
-  if (pl.tiles) {
-    // pl.heads KV heads at a time: their pages dequantized once into the
-    // workspace, then all row blocks of those heads over them, then their merge.
-    char *tiles = static_cast<char *>(workspace) + tiles_offset(pl, head_dim);
-    const unsigned npages = static_cast<unsigned>((seq_len + kPage - 1) / kPage);
-    a.tiles = tiles;
-    a.tile_head = static_cast<int64_t>(npages) * tile_stride(head_dim);
-    for (int h = 0; h < hkv; h += pl.heads) {
-      const int heads = std::min(pl.heads, hkv - h);
-      a.head0 = h;
-      a.total = pl.tper * heads;
-      a.grid = std::min(pl.grid, static_cast<int>(persistent_grid(a.total)));
-      a.xcd_perm = a.grid % 8 == 0 ? 1 : 0;
-      const dim3 cgrid(npages, static_cast<unsigned>(heads)), grid(static_cast<unsigned>(a.grid));
-      const dim3 mgrid(static_cast<unsigned>(pl.nbh * heads * kMergeSplit));
-      if (head_dim == 128) {
-        prefill_convert_kernel<<<cgrid, dim3(256), 0, s>>>(a, tiles);
-        if (std::min(pl.pages * heads / a.grid, pl.pages / pl.nbh) >= kWideMinPages)
-          prefill_tiles_kernel<128><<<grid, dim3(PW128::THREADS), 0, s>>>(a);
-        else
-          prefill_kernel<128, true><<<grid, dim3(PP::THREADS), 0, s>>>(a);
-        prefill_merge_kernel<128><<<mgrid, dim3(kMergeThreads), 0, s>>>(a);
-      } else {
-        prefill_convert256_kernel<<<cgrid, dim3(256), 0, s>>>(a, tiles);
-        prefill_tiles_kernel<256><<<grid, dim3(PW256::THREADS), 0, s>>>(a);
-        prefill_merge_kernel<256><<<mgrid, dim3(kMergeThreads), 0, s>>>(a);
-      }
-      const int rc = launch_status("k8v4_prefill_paged");
-      if (rc) return rc;
-    }
-    return K8V4_OK;
-  }
+  if (pl.tiles) return launch_over_tiles(a, pl, workspace, hkv, head_dim, s);
   if (head_dim == 128)
     prefill_kernel<128, false><<<dim3(static_cast<unsigned>(pl.grid)), dim3(Tile<128>::THREADS), 0, s>>>(a);
   else
@@ -2733,6 +2752,7 @@ extern "C" int k8v4_prefill_paged_batch(const void *q, int q_dtype, int64_t q_to
   const int ob = out_dtype == K8V4_F32 ? 4 : 2;
   std::vector<PrefillBatchArgs> launches;
   std::vector<int64_t> merge_blocks;
+  std::vector<std::pair<PrefillArgs, PrefillPlan>> singles;  // sequences worth tile images of their own
   int i = 0;
   while (i < nseq) {
     PrefillBatchArgs ba{};
@@ -2743,8 +2763,11 @@ extern "C" int k8v4_prefill_paged_batch(const void *q, int q_dtype, int64_t q_to
       K8V4_REQUIRE(plan_prefill(seq_lens[i], q_lens[i], hkv, head_dim, pl),
                    "sequence %d too large for one call (q_len %lld, seq_len %lld)", i,
                    static_cast<long long>(q_lens[i]), static_cast<long long>(seq_lens[i]));
-      const int k = ba.n++;
-      PrefillArgs &sa = ba.seq[k];
+      fit_workspace(pl, seq_lens[i], head_dim, workspace_bytes);
+      const bool over_tiles = pl.tiles && workspace_need(pl, seq_lens[i], head_dim) <= workspace_bytes;
+      if (over_tiles) singles.push_back({a, pl});
+      const int k = over_tiles ? 0 : ba.n++;
+      PrefillArgs &sa = over_tiles ? singles.back().first : ba.seq[k];
       sa = a;
       sa.q = a.q + tok0[i] * q_tok_stride;
       sa.out = static_cast<char *>(out) + tok0[i] * out_tok_stride * ob;
@@ -2754,6 +2777,7 @@ extern "C" int k8v4_prefill_paged_batch(const void *q, int q_dtype, int64_t q_to
       sa.nbh = pl.nbh;
       sa.tper = pl.tper;
       sa.cost = block_cost(head_dim);
+      if (over_tiles) continue;
       ba.step0[k] = static_cast<int>(steps);
       ba.block0[k] = static_cast<int>(blocks);
       steps += pl.total;
@@ -2761,7 +2785,7 @@ extern "C" int k8v4_prefill_paged_batch(const void *q, int q_dtype, int64_t q_to
       K8V4_REQUIRE(steps < (int64_t(1) << 30) && blocks * kMergeSplit < (int64_t(1) << 30),
                    "prefill batch too large for one launch");
     }
-    if (ba.n == 0) break;
+    if (ba.n == 0) continue;
     ba.step0[ba.n] = static_cast<int>(steps);
     ba.block0[ba.n] = static_cast<int>(blocks);
     const int64_t grid = persistent_grid(steps);
@@ -2772,6 +2796,10 @@ extern "C" int k8v4_prefill_paged_batch(const void *q, int q_dtype, int64_t q_to
     }
     launches.push_back(ba);
     merge_blocks.push_back(blocks);
+  }
+  for (const auto &one : singles) {
+    const int rc = launch_over_tiles(one.first, one.second, workspace, hkv, head_dim, s);
+    if (rc) return rc;
   }
   for (size_t j = 0; j < launches.size(); ++j) {
     const PrefillBatchArgs &ba = launches[j];

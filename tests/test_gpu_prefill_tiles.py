@@ -149,3 +149,39 @@ def test_batch_of_blocks_of_very_different_length(gpu_ops, d):
     for b, n in enumerate(lens):
         rows = slice(tok0[b], tok0[b] + q_lens[b])
         assert_close(out[rows].cpu().numpy(), _want(cache, q[rows], table[b], n), what="sequence %d" % b)
+
+
+@pytest.mark.parametrize("q_len,ctx", [(129, 26000), (150, 24001), (700, 3000), (1300, 0)])
+def test_d256_chunks_over_images_where_the_workspace_has_room(gpu_ops, q_len, ctx):
+    """Head dim 256, chunks that run over tile images if the workspace holds
+    them and in place otherwise, through the single and the batched entry."""
+    hkv, d, seq_len = 4, 256, q_len + ctx
+    lay = PageLayout(hkv, d)
+    assert not gpu_ops.prefill_uses_tiles(seq_len, q_len, hkv, d)
+    gen = torch.Generator().manual_seed(q_len + ctx)
+    lens = [seq_len, 200]
+    pool = sum(-(-n // PAGE) for n in lens) + 3
+    cache = Cache(pool, lay)
+    table = random_tables(gen, lens, pool)
+    for b, n in enumerate(lens):
+        fill_sequence(gpu_ops, cache, gen, table[b], n)
+    q = seeded_normal(gen, (q_len + 20, lay.hq, d))
+    want = [_want(cache, q[:q_len], table[0], seq_len), _want(cache, q[q_len:], table[1], 200)]
+    batch = gpu_ops.prefill_batch_workspace_bytes(hkv, d)
+    full = gpu_ops.prefill_workspace_bytes(seq_len, q_len, hkv, d)
+    pages = -(-seq_len // PAGE)
+    assert full > pages * 66 * 1024  # with the images
+    for nbytes in (batch, max(batch, full)):
+        ws = torch.empty(nbytes // 4, dtype=torch.float32, device=DEV)
+        out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=DEV)
+        gpu_ops.prefill_paged(q[:q_len].to(DEV), *cache.region_args(), table[0].to(device=DEV, dtype=torch.int32),
+                              seq_len, 1, 1.0 / 16, out[:q_len], ws)
+        torch.cuda.synchronize()
+        assert_close(out[:q_len].cpu().numpy(), want[0], what="single, %d bytes" % nbytes)
+        out.fill_(float("nan"))
+        gpu_ops.prefill_paged_batch(q.to(DEV), *cache.region_args(), table.to(DEV), [0, q_len], [q_len, 20], lens,
+                                    [0, 1], 1, 1.0 / 16, out, ws)
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        assert_close(got[:q_len], want[0], what="batch, %d bytes" % nbytes)
+        assert_close(got[q_len:], want[1], what="batch, second sequence")
