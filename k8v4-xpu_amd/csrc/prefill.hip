@@ -87,7 +87,7 @@ struct PrefillArgs {
   int total;     // steps of the launch (its heads * tper)
   int grid;      // persistent work-groups; work-group v takes steps [v*total/grid, (v+1)*total/grid)
   int xcd_perm;  // map ids so the work-groups of one XCD take adjacent work (grid % 8 == 0)
-  float *ws;     // partial states: [grid][2][rows][D + 2] floats
+  float *ws;     // partial states (part_index): [grid][2][rows * (D + 2)] floats
   int head0;     // KV head of step 0 (a launch covers heads head0 .. head0 + total / tper - 1)
   const char *tiles;  // dequantized tiles from head head0 on, [head][page][PP::BUF] (D = 128) or [page][PW256::IMG] bytes (null: convert in-kernel)
   int64_t tile_head;  // bytes of one head's tiles
@@ -289,6 +289,16 @@ __device__ __forceinline__ void store_out4(void *out, int dtype, int64_t idx, v4
     const v4h h = __builtin_convertvector(v, v4h);
     *reinterpret_cast<v4h *>(static_cast<_Float16 *>(out) + idx) = h;
   }
+}
+
+// Partial state of a piece of a row block: O [dt][j][hh][row][4] (dims 32 dt +
+// 8 j + 4 hh ..), m[row], l[row].  In this order the 16-byte stores of an
+// attention wave's lanes (one row each) and the loads of a merge wave's are
+// consecutive; as [row][D] each touched its own 128-byte line (merge kernel of a
+// whole prompt of 1,999 tokens, 4 heads of 128 dims: 20.8 -> 16.2 us).
+template <int ROWS>
+__device__ __forceinline__ int part_index(int dt, int j, int hh, int row) {
+  return ((8 * dt + 2 * j + hh) * ROWS + row) * 4;
 }
 
 // ---- balanced schedule (shared by the attention and merge kernels)
@@ -542,7 +552,7 @@ __device__ __forceinline__ void run_segment(const PrefillArgs &a, char *smem, in
         v4f o;
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = O[dt][4 * j + i] * ((i & 1) ? 1048576.f : 16777216.f) - cz;
-        *reinterpret_cast<v4f *>(part + lr * D + 32 * dt + 8 * j + 4 * hh) = o;
+        *reinterpret_cast<v4f *>(part + part_index<T::ROWS>(dt, j, hh, lr)) = o;
       }
     if (hh == 0) {
       part[T::ROWS * D + lr] = m_run;
@@ -1113,7 +1123,7 @@ __device__ __forceinline__ void run_segment_pp(const PrefillArgs &a, char *smem,
         v4f o;
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = 16.f * O[dt][4 * j + e];
-        *reinterpret_cast<v4f *>(part + lr * D + 32 * dt + 8 * j + 4 * hh) = o;
+        *reinterpret_cast<v4f *>(part + part_index<PP::ROWS>(dt, j, hh, lr)) = o;
       }
     if (hh == 0) {
       part[PP::ROWS * D + lr] = m_run;
@@ -1183,26 +1193,50 @@ __device__ __forceinline__ Segment last_segment(const PrefillArgs &a, int s0, in
   return g;
 }
 
-// ---- products of the tile-image paths, with the register files fixed: scores (and
-// the vector work on them) in VGPRs, O, the query and the operands read from
-// LDS in accumulation VGPRs; left to itself the compiler puts every product in
-// one file and copies or spills.  It does not see these as MFMAs: a result may
-// be read by another instruction kind only after mfma_settle() or four further
-// products.
+// ---- products of the tile-image paths, with the register files fixed: scores
+// (and the vector work on them) in VGPRs, O, the query and the operands read
+// from LDS in accumulation VGPRs; left to itself the compiler puts every
+// product in one file and copies or spills.  It does not see these as MFMAs, so
+// the distances it would keep are kept here: a result is read by another
+// instruction kind only after mfma_settle() or four further products, and an
+// operand that a vector instruction wrote is read two states later.  The
+// products outside the loops (EDGE) wait those two states themselves; the loops
+// hold every operand in its register, and a test checks the compiled code.
+template <bool EDGE = false>
 __device__ __forceinline__ void mfma_score0(v16f &d, v8h a, v8h b, const v16f &c) {
-  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "a"(b), "v"(c));
+  if constexpr (EDGE)
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "a"(b), "v"(c));
+  else
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "a"(b), "v"(c));
 }
+template <bool EDGE = false>
 __device__ __forceinline__ void mfma_score(v16f &d, v8h a, v8h b) {
-  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "a"(b));
+  if constexpr (EDGE)
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "a"(b));
+  else
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "a"(b));
 }
+// Query operand in VGPRs.
+template <bool EDGE = false>
 __device__ __forceinline__ void mfma_score0_v(v16f &d, v8h a, v8h b, const v16f &c) {
-  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "v"(b), "v"(c));
+  if constexpr (EDGE)
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "v"(b), "v"(c));
+  else
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "v"(b), "v"(c));
 }
+template <bool EDGE = false>
 __device__ __forceinline__ void mfma_score_v(v16f &d, v8h a, v8h b) {
-  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "v"(b));
+  if constexpr (EDGE)
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "a"(a), "v"(b));
 }
+template <bool EDGE = false>
 __device__ __forceinline__ void mfma_out(v16f &d, v8h a, v8h b) {
-  asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(d) : "a"(a), "v"(b));
+  if constexpr (EDGE)
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(d) : "a"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(d) : "a"(a), "v"(b));
 }
 __device__ __forceinline__ void mfma_settle() {
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -1482,11 +1516,11 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
   for (int f = 0; f < 16; ++f) {
     const v8h kf = k_frag(0, f);
     if (f == 0) {
-      mfma_score0(sA[0], kf, qf[0][f], minit[0]);
-      mfma_score0_v(sA[1], kf, qf[1][f], minit[1]);
+      mfma_score0<true>(sA[0], kf, qf[0][f], minit[0]);
+      mfma_score0_v<true>(sA[1], kf, qf[1][f], minit[1]);
     } else {
-      mfma_score(sA[0], kf, qf[0][f]);
-      mfma_score_v(sA[1], kf, qf[1][f]);
+      mfma_score<true>(sA[0], kf, qf[0][f]);
+      mfma_score_v<true>(sA[1], kf, qf[1][f]);
     }
   }
   mfma_settle();
@@ -1512,6 +1546,12 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
   asm volatile("s_waitcnt vmcnt(25) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
   for (int f = 0; f < AHEAD; ++f) fr[f] = k_frag(1, f);
+
+  // The query stays in its registers around the loop, as in the 128-dim path.
+  auto hold_query = [&]() {
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+a"(qf[0][ds]), "+v"(qf[1][ds]));
+  };
 
   // Iteration i of parity `par`: sc = S(i), sn = S(i + 1); pp = P(i - 1), pn = P(i).
   auto iteration = [&](int i, auto par_c, v16f (&sc)[2], v16f (&sn)[2], uint32_t (&pp)[2][8], uint32_t (&pn)[2][8]) {
@@ -1583,6 +1623,7 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
       if constexpr (s >= 53 && (s - 53) % 3 == 0) dma_v(i + 1, (s - 53) / 3);
       __builtin_amdgcn_sched_barrier(0);
     };
+    hold_query();
     mx[0] = mx[1] = -INFINITY;
     static_for<20>([&](auto sl) { slot(sl); });
     asm volatile("s_waitcnt vmcnt(17) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -1642,7 +1683,7 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
     const v8h vf = *reinterpret_cast<const v8h *>(vbase[f >> 2] + last_v + 4096 * (f & 3));
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
-      mfma_out(O[rt][f & 3], vf, f < 8 ? frag4(&pB[rt][4 * (f >> 2)]) : frag4(&pX[rt][4 * ((f >> 2) - 2)]));
+      mfma_out<true>(O[rt][f & 3], vf, f < 8 ? frag4(&pB[rt][4 * (f >> 2)]) : frag4(&pX[rt][4 * ((f >> 2) - 2)]));
   }
   // Row sums and zero-point terms of both halves of the keys.
   float l[2], cz[2];
@@ -1678,7 +1719,7 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
           v4f o;
 #pragma unroll
           for (int e = 0; e < 4; ++e) o[e] = O[rt][dt][4 * j + e] * ((e & 1) ? 1048576.f : 16777216.f) - cz[rt];
-          *reinterpret_cast<v4f *>(part + lr * D + 128 * half + 32 * dt + 8 * j + 4 * hh) = o;
+          *reinterpret_cast<v4f *>(part + part_index<PW256::ROWS>(4 * half + dt, j, hh, lr)) = o;
         }
       if (half == 0 && hh == 0) {
         part[PW256::ROWS * D + lr] = m_run[rt];
@@ -1853,14 +1894,24 @@ __device__ __forceinline__ void run_segment_wide(const PrefillArgs &a, char *sme
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
       if (f & 7)
-        mfma_score(sA[rt][f >> 3], kf, qf[rt][f & 7]);
+        mfma_score<true>(sA[rt][f >> 3], kf, qf[rt][f & 7]);
       else
-        mfma_score0(sA[rt][f >> 3], kf, qf[rt][f & 7], minit[rt]);
+        mfma_score0<true>(sA[rt][f >> 3], kf, qf[rt][f & 7], minit[rt]);
   }
 #pragma unroll
   for (int f = 0; f < AHEAD; ++f) fr[f] = v_frag(-1, f);
   mfma_settle();
   asm volatile("s_waitcnt vmcnt(9)\n\ts_barrier" ::: "memory");
+
+  // The query stays in its accumulation VGPRs around the loop (no copies there:
+  // they would cost an instruction per product and, unseen by the compiler as
+  // operands of an MFMA, come too close to it).
+  auto hold_query = [&]() {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+a"(qf[rt][ds]));
+  };
 
   // Iteration i: P = P(i - 1) -> P(i), O += V(i - 1) P(i - 1), sc = S(i), sn = S(i + 1).
   auto iteration = [&](int i, v16f (&sc)[2][2], v16f (&sn)[2][2]) {
@@ -1878,6 +1929,7 @@ __device__ __forceinline__ void run_segment_wide(const PrefillArgs &a, char *sme
         fr[f % AHEAD] = g < 16 ? v_frag(i - 1, g) : g < 32 ? k_frag(i + 1, g - 16) : v_frag(i, g - 32);
       }
     };
+    hold_query();
     float mx[2] = {-INFINITY, -INFINITY};
     static_for<8>([&](auto sl) {
       constexpr int s = decltype(sl)::value;
@@ -1969,7 +2021,7 @@ __device__ __forceinline__ void run_segment_wide(const PrefillArgs &a, char *sme
   for (int f = 0; f < 16; ++f) {
     const v8h vf = f < AHEAD ? fr[f] : v_frag(n - 1, f);
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) mfma_out(O[rt][f & 3], vf, p_frag(rt, f >> 2));
+    for (int rt = 0; rt < 2; ++rt) mfma_out<true>(O[rt][f & 3], vf, p_frag(rt, f >> 2));
   }
   // Nothing in flight when the ring is reused or the work-group ends.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1991,7 +2043,7 @@ __device__ __forceinline__ void run_segment_wide(const PrefillArgs &a, char *sme
           v4f o;
 #pragma unroll
           for (int e = 0; e < 4; ++e) o[e] = 16.f * O[rt][dt][4 * j + e];
-          *reinterpret_cast<v4f *>(part + lr * D + 32 * dt + 8 * j + 4 * hh) = o;
+          *reinterpret_cast<v4f *>(part + part_index<PW128::ROWS>(dt, j, hh, lr)) = o;
         }
       if (hh == 0) {
         part[PW128::ROWS * D + lr] = m_run[rt];
@@ -2156,16 +2208,14 @@ __global__ __launch_bounds__(256) void prefill_convert256_kernel(PrefillArgs a, 
 }
 
 // Finishes the blocks split between work-groups: kMergeSplit work-groups of
-// kMergeThreads per block (a launch then fills the chip), kMergeTPR<D>
-// threads per row, 32 dims each.  The pieces are folded in one pass with an
-// online rescale, their states loaded kMergeU at a time (all loads of a
-// round in flight together: the merge is a chain of round trips, not a
-// bandwidth problem).
-constexpr int kMergeSplit = 8;
+// kMergeThreads per block (a launch then fills the chip), each 128 rows by 16
+// dims, a row per thread (a call of 8 short chunks: 65.3 us with 32 dims, 54.6
+// with 16, 54.9 with 8).  The pieces are folded in one pass with an online
+// rescale, their states loaded kMergeU at a time (all loads of a round in
+// flight together: the merge is a chain of round trips).
+constexpr int kMergeSplit = 16;
 constexpr int kMergeThreads = 128;
 constexpr int kMergeU = 4;
-template <int D>
-constexpr int kMergeTPR = kMergeThreads * kMergeSplit / Tile<D>::ROWS;
 
 // Steps of row blocks 0 .. rb - 1 of one KV head (wave-uniform).
 __device__ __forceinline__ int steps_before_block(const PrefillArgs &a, int rb, int lane) {
@@ -2183,12 +2233,12 @@ __device__ __forceinline__ int steps_before_block(const PrefillArgs &a, int rb, 
 template <int D>
 __device__ __forceinline__ void merge_block(const PrefillArgs &a, const PrefillArgs &sa, int h, int rb, int start,
                                             int part) {
-  constexpr int R = Tile<D>::ROWS, TPR = kMergeTPR<D>, DT = D / TPR;  // DT = 32 dims per thread
-  static_assert(DT == 32, "32 dims per merge thread");
+  constexpr int R = Tile<D>::ROWS, DT = 16, SUBS = D / DT;
+  static_assert(R * SUBS == kMergeSplit * kMergeThreads && R % kMergeThreads == 0, "128 rows by 16 dims per work-group");
   const int n = block_pages(sa, rb);
   const int va = range_owner(a, start + sa.cost), vb = range_owner(a, start + sa.cost + n - 1);
   if (va == vb) return;  // one work-group did the whole block
-  const int lr = part * (R / kMergeSplit) + threadIdx.x / TPR, sub = threadIdx.x % TPR;
+  const int sub = part % SUBS, lr = part / SUBS * kMergeThreads + threadIdx.x;
   const int row = rb * R + lr;
   if (row >= sa.q_len * 6) return;
   float M = -INFINITY, l = 0.f;
@@ -2196,26 +2246,28 @@ __device__ __forceinline__ void merge_block(const PrefillArgs &a, const PrefillA
 #pragma unroll
   for (int e = 0; e < DT / 4; ++e) o[e] = (v4f){0.f, 0.f, 0.f, 0.f};
   for (int v0 = va; v0 <= vb; v0 += kMergeU) {
-    // This round's pieces (past vb: the last piece again, dropped below).
+    // This round's pieces (none past vb).
     float mu[kMergeU], lu[kMergeU];
     v4f ou[kMergeU][DT / 4];
 #pragma unroll
     for (int u = 0; u < kMergeU; ++u) {
-      const int v = min(v0 + u, vb);
+      const int v = v0 + u;
+      mu[u] = -INFINITY;
+      lu[u] = 0.f;
+#pragma unroll
+      for (int e = 0; e < DT / 4; ++e) ou[u][e] = (v4f)0.f;
+      if (v > vb) continue;
       const int slot = range_start(a, v) >= start ? 0 : 1;
       const float *pp = a.ws + (static_cast<int64_t>(v) * 2 + slot) * R * (D + 2);
       mu[u] = pp[R * D + lr];
       lu[u] = pp[R * D + R + lr];
-      const v4f *src = reinterpret_cast<const v4f *>(pp + lr * D + sub * DT);
 #pragma unroll
-      for (int e = 0; e < DT / 4; ++e) ou[u][e] = src[e];
+      for (int e = 0; e < DT / 4; ++e)
+        ou[u][e] = *reinterpret_cast<const v4f *>(pp + part_index<R>(sub >> 1, 2 * (sub & 1) + (e >> 1), e & 1, lr));
     }
     float Mn = M;
 #pragma unroll
-    for (int u = 0; u < kMergeU; ++u) {
-      if (v0 + u > vb) mu[u] = -INFINITY;
-      Mn = fmaxf(Mn, mu[u]);
-    }
+    for (int u = 0; u < kMergeU; ++u) Mn = fmaxf(Mn, mu[u]);
     if (Mn == -INFINITY) continue;  // no key seen yet by this row
     const float keep = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
     l *= keep;
@@ -2223,8 +2275,8 @@ __device__ __forceinline__ void merge_block(const PrefillArgs &a, const PrefillA
     for (int e = 0; e < DT / 4; ++e) o[e] *= keep;
 #pragma unroll
     for (int u = 0; u < kMergeU; ++u) {
-      // A piece that saw no key of this row (m = -inf) and the repeats past
-      // vb are selected away, not multiplied by zero.
+      // A piece that saw no key of this row (m = -inf) is selected away, not
+      // multiplied by zero.
       const bool on = mu[u] != -INFINITY;
       const float wgt = __builtin_amdgcn_exp2f(mu[u] - Mn);
       l = on ? l + wgt * lu[u] : l;
