@@ -2420,9 +2420,12 @@ constexpr int64_t kMinSteps = 4;
 // What a row block costs besides its pages, in page steps.  8 chunks of 17-128
 // tokens over 0.1K-8K (4 heads of 128 dims): 109 us with 0, 82, 70, 64, 63.0,
 // 63.7 us with 1, 2, 3, 4, 6; a whole prompt of 1,999 tokens 100 -> 69 us with
-// 4.  Head dim 256 (a page step takes longer): the same chunks 231 us with 0,
-// 149, 127, 127, 131 us with 1, 2, 3, 4.
-int block_cost(int head_dim) { return head_dim == 128 ? 4 : 2; }
+// 4, and over images of 4,224 tokens 155 -> 146 us with 6.  Head dim 256 in
+// place (a page step takes longer): the same chunks 231 us with 0, 149, 127,
+// 127, 131 us with 1, 2, 3, 4; over images (whole prompts of 2,000 tokens, 4
+// heads / 4,224, 2 heads): 139 / 237 us with 2, 112 / 182 with 4, 98 / 151 with
+// 8, 98 / 154 with 12.
+int block_cost(int head_dim, bool tiles) { return head_dim == 128 ? (tiles ? 6 : 4) : (tiles ? 8 : 2); }
 
 int rows_per_block(int head_dim) { return head_dim == 128 ? Tile<128>::ROWS : Tile<256>::ROWS; }
 
@@ -2439,14 +2442,14 @@ bool tiles_pay_off(int64_t nbh, int64_t npages, int head_dim) {
   return head_dim == 128 || (9 * nbh - 62) * npages > 58600;
 }
 
-// Head dim 256, other calls of more than 128 tokens, if the workspace has room:
-// the images cost about 10 ns per (page, head) and 19 us a call, and save 10 ns
-// per (row block, page, head).  In place against over images: 512 tokens over
-// 7,777, 4 heads, 243 -> 148 us; 512 over 16,384, 2 heads, 249 -> 149; whole
-// prompt of 2,000, 4 heads, 174 -> 154; of 1,000 (pages - images = 1,516)
-// 75.6 -> 70.5; 512 over 100 (536) 48.7 -> 54.9.
+// Head dim 256, other calls of more than 128 tokens, if the workspace has room
+// (in place against over images, pages - images in brackets): 512 tokens over
+// 7,777, 4 heads [11,500], 243 -> 135 us; 512 over 4,096, 2 heads [3,144],
+// 95.8 -> 63.3; whole prompt of 1,000, 4 heads [1,504], 66.0 -> 57.5; 150 over
+// 5,000, 2 heads [1,120], 52.2 -> 46.0; 512 over 100, 4 heads [552], 45.8 ->
+// 45.3; 300 over 300 [440], 43.8 -> 42.2.
 bool images_pay_off(int64_t nbh, int64_t pages, int64_t npages, int hkv, int head_dim) {
-  return head_dim == 256 && nbh > 6 && (pages - npages) * hkv > 1900;
+  return head_dim == 256 && nbh > 6 && (pages - npages) * hkv > 300;
 }
 
 int64_t tile_stride(int head_dim) { return head_dim == 128 ? PP::BUF : PW256::IMG; }
@@ -2503,15 +2506,17 @@ bool plan_prefill(int64_t seq_len, int64_t q_len, int hkv, int head_dim, Prefill
     const int64_t tok_hi = std::min<int64_t>(q_len - 1, (rb * R + R - 1) / 6);
     pages += (seq_len - q_len + tok_hi + 1 + 63) / 64;
   }
-  const int64_t tper = pages + nbh * block_cost(head_dim);
+  const bool alone = tiles_pay_off(nbh, (seq_len + kPage - 1) / kPage, head_dim);
+  const bool tiles = alone || images_pay_off(nbh, pages, (seq_len + kPage - 1) / kPage, hkv, head_dim);
+  const int64_t tper = pages + nbh * block_cost(head_dim, tiles);
   const int64_t total = tper * hkv;
   if (nbh < 1 || total < 1 || total >= (int64_t(1) << 31) / 2) return false;
   pl.nbh = static_cast<int>(nbh);
   pl.tper = static_cast<int>(tper);
   pl.total = static_cast<int>(total);
   pl.pages = pages;
-  pl.alone = tiles_pay_off(nbh, (seq_len + kPage - 1) / kPage, head_dim);
-  pl.tiles = pl.alone || images_pay_off(nbh, pages, (seq_len + kPage - 1) / kPage, hkv, head_dim);
+  pl.alone = alone;
+  pl.tiles = tiles;
   // The grid of the launch that runs: with tile images over the steps of
   // pl.heads KV heads, else over all heads.
   pl.heads = pl.tiles ? heads_per_launch((seq_len + kPage - 1) / kPage, hkv, head_dim) : hkv;
@@ -2550,6 +2555,8 @@ void fit_workspace(PrefillPlan &pl, int64_t seq_len, int head_dim, int64_t bytes
   if (workspace_need(pl, seq_len, head_dim) > bytes && pl.tiles && !pl.alone) {
     pl.tiles = false;
     pl.heads = pl.total / pl.tper;  // in place: all heads in one launch
+    pl.tper = static_cast<int>(pl.pages + pl.nbh * block_cost(head_dim, false));
+    pl.total = pl.tper * pl.heads;
     pl.grid = static_cast<int>(persistent_grid(pl.total));
   }
   if (workspace_need(pl, seq_len, head_dim) > bytes) pl.grid = static_cast<int>(least_grid(pl.pages * pl.heads));
@@ -2717,7 +2724,7 @@ extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stri
   a.rows = rows_per_block(head_dim);
   a.nbh = pl.nbh;
   a.tper = pl.tper;
-  a.cost = block_cost(head_dim);
+  a.cost = block_cost(head_dim, pl.tiles);
   a.total = pl.total;
   a.grid = pl.grid;
   a.xcd_perm = pl.grid % 8 == 0 ? 1 : 0;
@@ -2828,7 +2835,7 @@ extern "C" int k8v4_prefill_paged_batch(const void *q, int q_dtype, int64_t q_to
       sa.seq_len = static_cast<int>(seq_lens[i]);
       sa.nbh = pl.nbh;
       sa.tper = pl.tper;
-      sa.cost = block_cost(head_dim);
+      sa.cost = block_cost(head_dim, pl.tiles);
       if (over_tiles) continue;
       ba.step0[k] = static_cast<int>(steps);
       ba.block0[k] = static_cast<int>(blocks);
