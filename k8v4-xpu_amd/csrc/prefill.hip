@@ -315,12 +315,23 @@ __device__ __forceinline__ int part_index(int dt, int j, int hh, int row) {
 // pages alone counted, a work-group that drew eight one-page blocks took
 // several times as long as one with eight pages of one block (block_cost()).
 
-__device__ __forceinline__ int block_pages(const PrefillArgs &a, int rb) {
+__host__ __device__ __forceinline__ int block_pages(const PrefillArgs &a, int rb) {
   const int tok_hi = min(a.q_len - 1, (rb * a.rows + a.rows - 1) / 6);
   return (a.seq_len - a.q_len + tok_hi + 1 + 63) / 64;
 }
 
-__device__ __forceinline__ int block_steps(const PrefillArgs &a, int rb) { return a.cost + block_pages(a, rb); }
+__host__ __device__ __forceinline__ int block_steps(const PrefillArgs &a, int rb) { return a.cost + block_pages(a, rb); }
+
+// What a work-group at step s of its range (up to step s1) does in the block of
+// `a` that holds s, whose steps start at `base` and whose pages are n: pages
+// [p_lo, p_hi) (none if equal), then on to step `end`, past s.
+struct Piece {
+  int p_lo, p_hi, end;
+};
+__host__ __device__ __forceinline__ Piece piece_at(const PrefillArgs &a, int base, int n, int s, int s1) {
+  const int end = min(s1, base + a.cost + n);
+  return Piece{max(0, s - base - a.cost), max(0, end - base - a.cost), end};
+}
 
 // Block of one head that contains step sp (0 <= sp < tper), and the steps of
 // the blocks before it.  Wave-uniform.
@@ -348,12 +359,19 @@ __device__ __forceinline__ void locate_block(const PrefillArgs &a, int sp, int l
   }
 }
 
-__device__ __forceinline__ int range_start(const PrefillArgs &a, int v) {
+__host__ __device__ __forceinline__ int range_start(const PrefillArgs &a, int v) {
   return static_cast<int>(static_cast<int64_t>(v) * a.total / a.grid);
 }
 // Work-group whose range holds step s.
-__device__ __forceinline__ int range_owner(const PrefillArgs &a, int s) {
+__host__ __device__ __forceinline__ int range_owner(const PrefillArgs &a, int s) {
   return static_cast<int>(((static_cast<int64_t>(s) + 1) * a.grid - 1) / a.total);
+}
+// First and last work-group with pages of a block of `sa` whose steps start at
+// `start` and whose pages are n; `a` holds the launch's total and grid.
+__host__ __device__ __forceinline__ void page_owners(const PrefillArgs &a, const PrefillArgs &sa, int start, int n,
+                                                     int &va, int &vb) {
+  va = range_owner(a, start + sa.cost);
+  vb = range_owner(a, start + sa.cost + n - 1);
 }
 
 // One segment: pages [p_lo, p_hi) of row block rb of KV head h.  `part` is
@@ -2119,8 +2137,7 @@ prefill_kernel(PrefillArgs a) {
     locate_block(a, s - hl * a.tper, lane, rb, before);
     const int base = hl * a.tper + before;
     const int n = block_pages(a, rb);
-    const int end = min(s1, base + a.cost + n);
-    const int p_lo = max(0, s - base - a.cost), p_hi = max(0, end - base - a.cost);
+    const auto [p_lo, p_hi, end] = piece_at(a, base, n, s, s1);
     s = end;
     if (p_lo == p_hi) continue;
     float *part = nullptr;
@@ -2236,7 +2253,8 @@ __device__ __forceinline__ void merge_block(const PrefillArgs &a, const PrefillA
   constexpr int R = Tile<D>::ROWS, DT = 16, SUBS = D / DT;
   static_assert(R * SUBS == kMergeSplit * kMergeThreads && R % kMergeThreads == 0, "128 rows by 16 dims per work-group");
   const int n = block_pages(sa, rb);
-  const int va = range_owner(a, start + sa.cost), vb = range_owner(a, start + sa.cost + n - 1);
+  int va, vb;
+  page_owners(a, sa, start, n, va, vb);
   if (va == vb) return;  // one work-group did the whole block
   const int sub = part % SUBS, lr = part / SUBS * kMergeThreads + threadIdx.x;
   const int row = rb * R + lr;
@@ -2372,8 +2390,7 @@ prefill_batch_kernel(PrefillBatchArgs ba) {
     locate_block(sa, s - first - h * sa.tper, lane, rb, before);
     const int base = first + h * sa.tper + before;
     const int n = block_pages(sa, rb);
-    const int end = min(s1, base + a.cost + n);
-    const int p_lo = max(0, s - base - a.cost), p_hi = max(0, end - base - a.cost);
+    const auto [p_lo, p_hi, end] = piece_at(sa, base, n, s, s1);
     s = end;
     if (p_lo == p_hi) continue;
     float *part = nullptr;
@@ -2543,22 +2560,24 @@ int64_t workspace_size(const PrefillPlan &pl, int64_t seq_len, int hkv, int head
   return (partial_bytes(static_cast<int>(persistent_grid(static_cast<int64_t>(pl.tper) * hkv)), head_dim) + 255) / 256 * 256 +
          pages * tile_stride(head_dim);
 }
+// The plan of a call whose pages are converted in place, all heads in one launch.
+void plan_in_place(PrefillPlan &pl, int hkv, int head_dim) {
+  pl.tiles = false;
+  pl.heads = hkv;
+  pl.tper = static_cast<int>(pl.pages + pl.nbh * block_cost(head_dim, false));
+  pl.total = pl.tper * hkv;
+  pl.grid = static_cast<int>(persistent_grid(pl.total));
+}
 // A smaller workspace than workspace_size() still serves a call that fits it
 // with fewer heads a launch, down to one, in place where the call is not one
 // that always runs over tile images, and with the work-groups counted by page
 // steps alone.
-void fit_workspace(PrefillPlan &pl, int64_t seq_len, int head_dim, int64_t bytes) {
+void fit_workspace(PrefillPlan &pl, int64_t seq_len, int hkv, int head_dim, int64_t bytes) {
   while (pl.tiles && pl.heads > 1 && workspace_need(pl, seq_len, head_dim) > bytes) {
     --pl.heads;
     pl.grid = static_cast<int>(persistent_grid(static_cast<int64_t>(pl.tper) * pl.heads));
   }
-  if (workspace_need(pl, seq_len, head_dim) > bytes && pl.tiles && !pl.alone) {
-    pl.tiles = false;
-    pl.heads = pl.total / pl.tper;  // in place: all heads in one launch
-    pl.tper = static_cast<int>(pl.pages + pl.nbh * block_cost(head_dim, false));
-    pl.total = pl.tper * pl.heads;
-    pl.grid = static_cast<int>(persistent_grid(pl.total));
-  }
+  if (workspace_need(pl, seq_len, head_dim) > bytes && pl.tiles && !pl.alone) plan_in_place(pl, hkv, head_dim);
   if (workspace_need(pl, seq_len, head_dim) > bytes) pl.grid = static_cast<int>(least_grid(pl.pages * pl.heads));
 }
 
@@ -2620,6 +2639,67 @@ int launch_over_tiles(PrefillArgs a, const PrefillPlan &pl, void *workspace, int
     }
     const int rc = launch_status("k8v4_prefill_paged");
     if (rc) return rc;
+  }
+  return K8V4_OK;
+}
+
+// Launches of up to kBatchMax non-empty sequences each, one after another on
+// the stream (each launch reuses the workspace after the previous one), and the
+// sequences that run over tile images of their own before them.  Everything is
+// planned and checked before the first launch is enqueued, so a rejected call
+// launches nothing.
+struct BatchPlan {
+  std::vector<PrefillBatchArgs> launches;
+  std::vector<std::pair<PrefillArgs, PrefillPlan>> singles;
+};
+int plan_batch(const PrefillArgs &a, const int32_t *block_table, int64_t bt_stride, int nseq, const int64_t *tok0,
+               const int64_t *q_lens, const int64_t *seq_lens, const int64_t *rows, int head_dim,
+               int64_t workspace_bytes, BatchPlan &plan) {
+  const int ob = a.out_dtype == K8V4_F32 ? 4 : 2;
+  int i = 0;
+  while (i < nseq) {
+    PrefillBatchArgs ba{};
+    int64_t steps = 0, blocks = 0;
+    for (; i < nseq && ba.n < kBatchMax; ++i) {
+      if (q_lens[i] == 0) continue;
+      PrefillPlan pl;
+      K8V4_REQUIRE(plan_prefill(seq_lens[i], q_lens[i], a.hkv, head_dim, pl),
+                   "sequence %d too large for one call (q_len %lld, seq_len %lld)", i,
+                   static_cast<long long>(q_lens[i]), static_cast<long long>(seq_lens[i]));
+      fit_workspace(pl, seq_lens[i], a.hkv, head_dim, workspace_bytes);
+      const bool over_tiles = pl.tiles && workspace_need(pl, seq_lens[i], head_dim) <= workspace_bytes;
+      // The rest of the launch is planned in place too: one fixed cost per block.
+      if (!over_tiles) plan_in_place(pl, a.hkv, head_dim);
+      if (over_tiles) plan.singles.push_back({a, pl});
+      const int k = over_tiles ? 0 : ba.n++;
+      PrefillArgs &sa = over_tiles ? plan.singles.back().first : ba.seq[k];
+      sa = a;
+      sa.q = a.q + tok0[i] * a.q_tok_stride;
+      sa.out = static_cast<char *>(a.out) + tok0[i] * a.out_tok_stride * ob;
+      sa.block_row = block_table + rows[i] * bt_stride;
+      sa.q_len = static_cast<int>(q_lens[i]);
+      sa.seq_len = static_cast<int>(seq_lens[i]);
+      sa.nbh = pl.nbh;
+      sa.tper = pl.tper;
+      sa.cost = block_cost(head_dim, pl.tiles);
+      if (over_tiles) continue;
+      ba.step0[k] = static_cast<int>(steps);
+      ba.block0[k] = static_cast<int>(blocks);
+      steps += pl.total;
+      blocks += static_cast<int64_t>(pl.nbh) * a.hkv;
+      K8V4_REQUIRE(steps < (int64_t(1) << 30) && blocks * kMergeSplit < (int64_t(1) << 30),
+                   "prefill batch too large for one launch");
+    }
+    if (ba.n == 0) continue;
+    ba.step0[ba.n] = static_cast<int>(steps);
+    ba.block0[ba.n] = static_cast<int>(blocks);
+    const int64_t grid = persistent_grid(steps);
+    for (int k = 0; k < ba.n; ++k) {
+      ba.seq[k].total = static_cast<int>(steps);
+      ba.seq[k].grid = static_cast<int>(grid);
+      ba.seq[k].xcd_perm = grid % 8 == 0 ? 1 : 0;
+    }
+    plan.launches.push_back(ba);
   }
   return K8V4_OK;
 }
@@ -2712,7 +2792,7 @@ extern "C" int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stri
   PrefillPlan pl;
   K8V4_REQUIRE(plan_prefill(seq_len, q_len, hkv, head_dim, pl), "prefill too large for one call (q_len %lld, seq_len %lld)",
                static_cast<long long>(q_len), static_cast<long long>(seq_len));
-  fit_workspace(pl, seq_len, head_dim, workspace_bytes);
+  fit_workspace(pl, seq_len, hkv, head_dim, workspace_bytes);
   const int64_t need = workspace_need(pl, seq_len, head_dim);
   K8V4_REQUIRE(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
                "prefill workspace must be a 16-byte aligned device buffer");
@@ -2804,66 +2884,18 @@ extern "C" int k8v4_prefill_paged_batch(const void *q, int q_dtype, int64_t q_to
   a.head0 = 0;
   a.tiles = nullptr;
   auto s = static_cast<hipStream_t>(stream);
-  // Launches of up to kBatchMax non-empty sequences each, one after another
-  // on the stream (each launch reuses the workspace after the previous one).
-  // All of them are planned and checked before the first is enqueued, so a
-  // rejected call launches nothing.
-  const int ob = out_dtype == K8V4_F32 ? 4 : 2;
-  std::vector<PrefillBatchArgs> launches;
-  std::vector<int64_t> merge_blocks;
-  std::vector<std::pair<PrefillArgs, PrefillPlan>> singles;  // sequences worth tile images of their own
-  int i = 0;
-  while (i < nseq) {
-    PrefillBatchArgs ba{};
-    int64_t steps = 0, blocks = 0;
-    for (; i < nseq && ba.n < kBatchMax; ++i) {
-      if (q_lens[i] == 0) continue;
-      PrefillPlan pl;
-      K8V4_REQUIRE(plan_prefill(seq_lens[i], q_lens[i], hkv, head_dim, pl),
-                   "sequence %d too large for one call (q_len %lld, seq_len %lld)", i,
-                   static_cast<long long>(q_lens[i]), static_cast<long long>(seq_lens[i]));
-      fit_workspace(pl, seq_lens[i], head_dim, workspace_bytes);
-      const bool over_tiles = pl.tiles && workspace_need(pl, seq_lens[i], head_dim) <= workspace_bytes;
-      if (over_tiles) singles.push_back({a, pl});
-      const int k = over_tiles ? 0 : ba.n++;
-      PrefillArgs &sa = over_tiles ? singles.back().first : ba.seq[k];
-      sa = a;
-      sa.q = a.q + tok0[i] * q_tok_stride;
-      sa.out = static_cast<char *>(out) + tok0[i] * out_tok_stride * ob;
-      sa.block_row = block_table + rows[i] * bt_stride;
-      sa.q_len = static_cast<int>(q_lens[i]);
-      sa.seq_len = static_cast<int>(seq_lens[i]);
-      sa.nbh = pl.nbh;
-      sa.tper = pl.tper;
-      sa.cost = block_cost(head_dim, pl.tiles);
-      if (over_tiles) continue;
-      ba.step0[k] = static_cast<int>(steps);
-      ba.block0[k] = static_cast<int>(blocks);
-      steps += pl.total;
-      blocks += static_cast<int64_t>(pl.nbh) * hkv;
-      K8V4_REQUIRE(steps < (int64_t(1) << 30) && blocks * kMergeSplit < (int64_t(1) << 30),
-                   "prefill batch too large for one launch");
-    }
-    if (ba.n == 0) continue;
-    ba.step0[ba.n] = static_cast<int>(steps);
-    ba.block0[ba.n] = static_cast<int>(blocks);
-    const int64_t grid = persistent_grid(steps);
-    for (int k = 0; k < ba.n; ++k) {
-      ba.seq[k].total = static_cast<int>(steps);
-      ba.seq[k].grid = static_cast<int>(grid);
-      ba.seq[k].xcd_perm = grid % 8 == 0 ? 1 : 0;
-    }
-    launches.push_back(ba);
-    merge_blocks.push_back(blocks);
+  BatchPlan plan;
+  {
+    const int rc = plan_batch(a, block_table, bt_stride, nseq, tok0, q_lens, seq_lens, rows, head_dim, workspace_bytes, plan);
+    if (rc) return rc;
   }
-  for (const auto &one : singles) {
+  for (const auto &one : plan.singles) {
     const int rc = launch_over_tiles(one.first, one.second, workspace, hkv, head_dim, s);
     if (rc) return rc;
   }
-  for (size_t j = 0; j < launches.size(); ++j) {
-    const PrefillBatchArgs &ba = launches[j];
+  for (const PrefillBatchArgs &ba : plan.launches) {
     const dim3 grid(static_cast<unsigned>(ba.seq[0].grid));
-    const dim3 mgrid(static_cast<unsigned>(merge_blocks[j] * kMergeSplit));
+    const dim3 mgrid(static_cast<unsigned>(ba.block0[ba.n]) * kMergeSplit);
     if (head_dim == 128) {
       prefill_batch_kernel<128><<<grid, dim3(Tile<128>::THREADS), 0, s>>>(ba);
       prefill_batch_merge_kernel<128><<<mgrid, dim3(kMergeThreads), 0, s>>>(ba);

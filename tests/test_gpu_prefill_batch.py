@@ -20,7 +20,8 @@ import torch
 from gpu_cases import DEV, Cache, assert_close, fill_sequence, random_tables, seeded_normal
 from k8v4_v030.layout import PAGE, PageLayout
 from k8v4_v030.prefill import hip_prefill
-from oracle import attention
+from oracle import attention, torch_cpu
+from oracle.paged import Geometry
 
 pytestmark = pytest.mark.gpu
 
@@ -129,3 +130,25 @@ def test_empty_sequences_are_skipped_and_rows_checked(gpu_ops):
     with pytest.raises(RuntimeError, match="sequence rows outside the query"):
         gpu_ops.prefill_paged_batch(q.to(DEV), *cache.region_args(), table.to(device=DEV, dtype=torch.int32),
                                     [q.shape[0] - 1], [2], [8], [0], 1, 0.1, out)
+
+
+@pytest.mark.parametrize("order", [(0, 1, 2), (2, 1, 0)])
+@pytest.mark.parametrize("hkv,d,q_lens,seq_lens", [
+    (4, 128, [64, 170, 20], [2048, 16554, 300]), (2, 256, [64, 512, 20], [2048, 30000, 300]),
+])
+def test_a_chunk_whose_images_do_not_fit_shares_the_launch(gpu_ops, hkv, d, q_lens, seq_lens, order):
+    """The least workspace holds no tile images of the long chunk, which the
+    single entry would always run over images: its pages are converted in place
+    beside the short chunks', before or after them in the launch."""
+    print("prefill batch, long beside short, hkv=%d d=%d %s" % (hkv, d, order), flush=True)
+    q_lens, seq_lens = [q_lens[i] for i in order], [seq_lens[i] for i in order]
+    lay = PageLayout(hkv, d)
+    gen = torch.Generator().manual_seed(31 * d + order[0])
+    assert gpu_ops.prefill_uses_tiles(seq_lens[1], q_lens[1], hkv, d)
+    assert gpu_ops.prefill_workspace_bytes(seq_lens[1], q_lens[1], hkv, d) > gpu_ops.prefill_batch_workspace_bytes(hkv, d)
+    cache, table, q, tok0, rows = _setup(gpu_ops, gen, lay, q_lens, seq_lens)
+    got = _batch(gpu_ops, cache, table, q, tok0, q_lens, seq_lens, rows)
+    views = torch_cpu.region_views(torch.from_numpy(cache.blob().copy()), Geometry(hkv, d))
+    for t, ql, sl, r in zip(tok0, q_lens, seq_lens, rows):
+        want = torch_cpu.prefill(views, q[t : t + ql], table[r].long(), sl, 1.0 / math.sqrt(d)).numpy()
+        assert_close(got[t : t + ql], want, what="q %d over %d" % (ql, sl))
