@@ -1220,12 +1220,18 @@ __device__ __forceinline__ Segment last_segment(const PrefillArgs &a, int s0, in
 // operand that a vector instruction wrote is read two states later.  The
 // products outside the loops (EDGE) wait those two states themselves; the loops
 // hold every operand in its register, and a test checks the compiled code.
+// A product goes on reading a start value that is not its result's register
+// after it was issued, so nothing may overwrite that for 15 states: it is an
+// operand the product also "writes", which the compiler then keeps for the next
+// page in those registers (as a plain input it took a copy and reused that at
+// once; accumulating in place instead costs 32 or 64 moves a page, and copies
+// of half-finished tuples at 128 dims).
 template <bool EDGE = false>
-__device__ __forceinline__ void mfma_score0(v16f &d, v8h a, v8h b, const v16f &c) {
+__device__ __forceinline__ void mfma_score0(v16f &d, v8h a, v8h b, v16f &c) {
   if constexpr (EDGE)
-    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "a"(b), "v"(c));
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %2, %3, %1" : "=&v"(d), "+v"(c) : "a"(a), "a"(b));
   else
-    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "a"(b), "v"(c));
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %2, %3, %1" : "=&v"(d), "+v"(c) : "a"(a), "a"(b));
 }
 template <bool EDGE = false>
 __device__ __forceinline__ void mfma_score(v16f &d, v8h a, v8h b) {
@@ -1236,11 +1242,11 @@ __device__ __forceinline__ void mfma_score(v16f &d, v8h a, v8h b) {
 }
 // Query operand in VGPRs.
 template <bool EDGE = false>
-__device__ __forceinline__ void mfma_score0_v(v16f &d, v8h a, v8h b, const v16f &c) {
+__device__ __forceinline__ void mfma_score0_v(v16f &d, v8h a, v8h b, v16f &c) {
   if constexpr (EDGE)
-    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "v"(b), "v"(c));
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %2, %3, %1" : "=&v"(d), "+v"(c) : "a"(a), "v"(b));
   else
-    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(d) : "a"(a), "v"(b), "v"(c));
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %2, %3, %1" : "=&v"(d), "+v"(c) : "a"(a), "v"(b));
 }
 template <bool EDGE = false>
 __device__ __forceinline__ void mfma_score_v(v16f &d, v8h a, v8h b) {
