@@ -227,9 +227,13 @@ int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stride, const i
  * take up to 10 non-empty sequences, whose (KV head, row block) work shares
  * the persistent work-groups of one launch; more sequences take more
  * launches, in order, on the stream.  Pages are dequantized in the kernel
- * (no per-head tile pre-pass), which suits short chunks; a chunk that
- * k8v4_prefill_paged would serve from tile images runs that way, by itself,
- * if the workspace has room for it.  The same bottom-right causal rule,
+ * (no per-head tile pre-pass), which suits short chunks.  A chunk that
+ * k8v4_prefill_paged may serve from tile images runs that way, before the
+ * shared launches, if the workspace has room for it and that costs less than
+ * its part of a shared launch (a measured rule on the row blocks and the
+ * pages they read: images_in_batch() in csrc/prefill.hip; on 256 compute units
+ * from about 3,300 page steps beside one other sequence at head_dim 256, 41,000
+ * at head_dim 128).  The same bottom-right causal rule,
  * numerics and errors per sequence as k8v4_prefill_paged; q_lens[i] == 0
  * sequences are skipped; nseq == 0 is a no-op.  The library sees neither
  * the table's row count nor the token count of q and out: the caller keeps

@@ -2475,6 +2475,27 @@ bool images_pay_off(int64_t nbh, int64_t pages, int64_t npages, int hkv, int hea
   return head_dim == 256 && nbh > 6 && (pages - npages) * hkv > 300;
 }
 
+// The same choice for a sequence of a batched call.  Alone in its call it runs as
+// through the single entry (head dim 128: from 24 row blocks on; 300 tokens over
+// 65,536, 8 blocks, took 301 us in place, 373 over images).  Beside others its
+// own launches have to cost less than the page steps it adds to every work-group
+// of the shared one.  Head dim 256: they are worth about 19 steps, and the shared
+// launch itself 12, which is saved if none is left for it (in place / over images,
+// us per call of 2, 4 and 8 chunks): 8.1 steps (300 tokens over 2,300 in all, 4
+// heads) 108 / 126, 189 / 247, 344 / 494; 12.9 (512 / 4,608, 2 heads) 152 / 145,
+// 275 / 289, 515 / 577; 16.0 (150 / 16,384, 2 heads) 176 / 160, 315 / 313; 17.6
+// (1,000 / 2,000, 4 heads) 213 / 184, 386 / 363; 26 (512 / 4,608, 4 heads) 276 /
+// 202, 516 / 404, 987 / 812.  Head dim 128, 4 chunks: 12 blocks, 96 steps (500 /
+// 33,000, 4 heads) 879 / 1,018; 24 blocks, 190 steps (1,000 / 33,000) 1,702 /
+// 1,717; more blocks, 74 steps 715 / 779, 148 steps 1,397 / 1,413, 177 steps
+// 1,618 / 1,591, 368 steps 3,455 / 3,055.
+bool images_in_batch(const PrefillPlan &pl, int sequences, int hkv, int head_dim) {
+  if (!pl.tiles || (head_dim == 128 && pl.nbh < 24)) return false;
+  if (sequences == 1) return true;
+  const int64_t steps = pl.pages * hkv, cus = device_cus();
+  return head_dim == 128 ? steps >= 160 * cus : steps * sequences >= (19 * sequences - 12) * cus;
+}
+
 int64_t tile_stride(int head_dim) { return head_dim == 128 ? PP::BUF : PW256::IMG; }
 
 // Persistent work-groups for a launch of `steps` steps: one per CU, each with
@@ -2662,6 +2683,7 @@ int plan_batch(const PrefillArgs &a, const int32_t *block_table, int64_t bt_stri
                const int64_t *q_lens, const int64_t *seq_lens, const int64_t *rows, int head_dim,
                int64_t workspace_bytes, BatchPlan &plan) {
   const int ob = a.out_dtype == K8V4_F32 ? 4 : 2;
+  const int sequences = nseq - static_cast<int>(std::count(q_lens, q_lens + nseq, 0));
   int i = 0;
   while (i < nseq) {
     PrefillBatchArgs ba{};
@@ -2672,8 +2694,11 @@ int plan_batch(const PrefillArgs &a, const int32_t *block_table, int64_t bt_stri
       K8V4_REQUIRE(plan_prefill(seq_lens[i], q_lens[i], a.hkv, head_dim, pl),
                    "sequence %d too large for one call (q_len %lld, seq_len %lld)", i,
                    static_cast<long long>(q_lens[i]), static_cast<long long>(seq_lens[i]));
-      fit_workspace(pl, seq_lens[i], a.hkv, head_dim, workspace_bytes);
-      const bool over_tiles = pl.tiles && workspace_need(pl, seq_lens[i], head_dim) <= workspace_bytes;
+      bool over_tiles = images_in_batch(pl, sequences, a.hkv, head_dim);
+      if (over_tiles) {
+        fit_workspace(pl, seq_lens[i], a.hkv, head_dim, workspace_bytes);
+        over_tiles = pl.tiles && workspace_need(pl, seq_lens[i], head_dim) <= workspace_bytes;
+      }
       // The rest of the launch is planned in place too: one fixed cost per block.
       if (!over_tiles) plan_in_place(pl, a.hkv, head_dim);
       if (over_tiles) plan.singles.push_back({a, pl});

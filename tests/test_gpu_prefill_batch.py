@@ -51,11 +51,11 @@ def _setup(ops, gen, lay, q_lens, seq_lens, ppb=1, gap=3, table_order=None):
     return cache, table, q, tok0, order
 
 
-def _batch(gpu_ops, cache, table, q, tok0, q_lens, seq_lens, rows, ppb=1, out_dtype=torch.float32):
+def _batch(gpu_ops, cache, table, q, tok0, q_lens, seq_lens, rows, ppb=1, out_dtype=torch.float32, workspace=None):
     out = torch.full(q.shape, float("nan"), dtype=out_dtype, device=DEV)
     scale = 1.0 / math.sqrt(cache.layout.head_dim)
     gpu_ops.prefill_paged_batch(q.to(DEV), *cache.region_args(), table.to(device=DEV, dtype=torch.int32), tok0,
-                                q_lens, seq_lens, rows, ppb, scale, out)
+                                q_lens, seq_lens, rows, ppb, scale, out, workspace=workspace)
     torch.cuda.synchronize()
     return out.float().cpu().numpy()
 
@@ -152,3 +152,25 @@ def test_a_chunk_whose_images_do_not_fit_shares_the_launch(gpu_ops, hkv, d, q_le
     for t, ql, sl, r in zip(tok0, q_lens, seq_lens, rows):
         want = torch_cpu.prefill(views, q[t : t + ql], table[r].long(), sl, 1.0 / math.sqrt(d)).numpy()
         assert_close(got[t : t + ql], want, what="q %d over %d" % (ql, sl))
+
+
+@pytest.mark.parametrize("hkv,d,q_lens,seq_lens", [
+    (4, 256, [400, 20], [4400, 200]),  # leaves the shared launch
+    (4, 256, [200, 20, 150], [900, 200, 2300]),  # share it with room for images
+    (2, 128, [1000, 0], [1100, 64]),  # alone in its call
+    (2, 128, [1000, 20], [1100, 64]),
+])
+def test_room_for_images_beside_other_sequences(gpu_ops, hkv, d, q_lens, seq_lens):
+    print("prefill batch with room for images, hkv=%d d=%d %s" % (hkv, d, q_lens), flush=True)
+    lay = PageLayout(hkv, d)
+    gen = torch.Generator().manual_seed(d + sum(q_lens))
+    cache, table, q, tok0, rows = _setup(gpu_ops, gen, lay, q_lens, seq_lens)
+    need = max([gpu_ops.prefill_batch_workspace_bytes(hkv, d)]
+               + [gpu_ops.prefill_workspace_bytes(s, n, hkv, d) for n, s in zip(q_lens, seq_lens)])
+    ws = torch.empty(need // 4, dtype=torch.float32, device=DEV)
+    got = _batch(gpu_ops, cache, table, q, tok0, q_lens, seq_lens, rows, workspace=ws)
+    views = torch_cpu.region_views(torch.from_numpy(cache.blob().copy()), Geometry(hkv, d))
+    for t, ql, sl, r in zip(tok0, q_lens, seq_lens, rows):
+        if ql:
+            want = torch_cpu.prefill(views, q[t : t + ql], table[r].long(), sl, 1.0 / math.sqrt(d)).numpy()
+            assert_close(got[t : t + ql], want, what="q %d over %d" % (ql, sl))
