@@ -145,10 +145,16 @@ def _on_gpu(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
+# The raw handle of torch.cuda.current_stream(dev), without building the Python
+# stream object around it: a private function, so where a torch lacks it the
+# public call serves.
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(dev: torch.device) -> int:
-    # The raw handle of torch.cuda.current_stream(dev), without building the
-    # Python stream object around it.
-    return torch._C._cuda_getCurrentRawStream(dev.index)
+    if _RAW_STREAM is None:
+        return int(torch.cuda.current_stream(dev).cuda_stream)
+    return _RAW_STREAM(dev.index)
 
 
 def _ptr(t: torch.Tensor) -> int:
