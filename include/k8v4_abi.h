@@ -232,7 +232,7 @@ int k8v4_prefill_paged(const void *q, int q_dtype, int64_t q_tok_stride, const i
  * shared launches, if the workspace has room for it and that costs less than
  * its part of a shared launch (a measured rule on the row blocks and the
  * pages they read: images_in_batch() in csrc/prefill.hip; on 256 compute units
- * from about 3,300 page steps beside one other sequence at head_dim 256, 41,000
+ * from about 1,800 page steps beside one other sequence at head_dim 256, 10,000
  * at head_dim 128).  The same bottom-right causal rule,
  * numerics and errors per sequence as k8v4_prefill_paged; q_lens[i] == 0
  * sequences are skipped; nseq == 0 is a no-op.  The library sees neither

@@ -2492,24 +2492,29 @@ bool images_pay_off(int64_t nbh, int64_t pages, int64_t npages, int hkv, int hea
 }
 
 // The same choice for a sequence of a batched call.  Alone in its call it runs as
-// through the single entry (head dim 128: from 24 row blocks on; 300 tokens over
-// 65,536, 8 blocks, took 301 us in place, 373 over images).  Beside others its
-// own launches have to cost less than the page steps it adds to every work-group
-// of the shared one.  Head dim 256: they are worth about 19 steps, and the shared
-// launch itself 12, which is saved if none is left for it (in place / over images,
-// us per call of 2, 4 and 8 chunks): 8.1 steps (300 tokens over 2,300 in all, 4
-// heads) 108 / 126, 189 / 247, 344 / 494; 12.9 (512 / 4,608, 2 heads) 152 / 145,
-// 275 / 289, 515 / 577; 16.0 (150 / 16,384, 2 heads) 176 / 160, 315 / 313; 17.6
-// (1,000 / 2,000, 4 heads) 213 / 184, 386 / 363; 26 (512 / 4,608, 4 heads) 276 /
-// 202, 516 / 404, 987 / 812.  Head dim 128, 4 chunks: 12 blocks, 96 steps (500 /
-// 33,000, 4 heads) 879 / 1,018; 24 blocks, 190 steps (1,000 / 33,000) 1,702 /
-// 1,717; more blocks, 74 steps 715 / 779, 148 steps 1,397 / 1,413, 177 steps
-// 1,618 / 1,591, 368 steps 3,455 / 3,055.
+// through the single entry (head dim 128: from 16 row blocks on; 300 tokens over
+// 65,536, 4 heads, 8 blocks, take 304 us in place, 341 over images).  Beside others
+// its own launches have to cost less than the page steps it adds to every
+// work-group of the shared one: they are worth about 12 steps (head dim 128, where
+// a step over images saves less: 100), and the shared launch itself 10 (120),
+// which is saved if none is left for it.  Over images / in place, us per call of
+// 2, 4 and 8 chunks:
+//   256 dims,  5.1 steps (150 tokens over 5,000, 2 heads)    84 /  73
+//              6.1       (1,000 over 0, 4 heads)            102 / 106   212 / 184   407 / 317
+//              8.0       (300 over 2,000, 4 heads)          101 / 110   196 / 187   376 / 333
+//              9.5       (300 over 5,000, 2 heads)           97 / 115   193 / 202   382 / 378
+//             11.2       (400 over 4,600, 2 heads)          106 / 132   209 / 237   417 / 442
+//             25.7       (512 over 4,096, 4 heads)          171 / 265   340 / 500   678 / 959
+//   128 dims, 35.0       (2,000 over 2,000, 4 heads)        214 / 203   427 / 373   879 / 723
+//             50.1       (1,000 over 8,000, 4 heads)        256 / 263   510 / 497 1,016 / 954
+//             74.0       (4,224 over 3,968, 2 heads)        361 / 380   719 / 726 1,464 / 1,428
+//             95.4       (1,000 over 32,000, 2 heads)       434 / 462   865 / 893 1,730 / 1,747
+//             95.9, 12 blocks (500 over 32,500, 4 heads)    460 / 460   929 / 881
 bool images_in_batch(const PrefillPlan &pl, int sequences, int hkv, int head_dim) {
-  if (!pl.tiles || (head_dim == 128 && pl.nbh < 24)) return false;
+  if (!pl.tiles || (head_dim == 128 && pl.nbh < 16)) return false;
   if (sequences == 1) return true;
-  const int64_t steps = pl.pages * hkv, cus = device_cus();
-  return head_dim == 128 ? steps >= 160 * cus : steps * sequences >= (19 * sequences - 12) * cus;
+  const int64_t own = head_dim == 128 ? 100 : 12, shared = head_dim == 128 ? 120 : 10;
+  return pl.pages * hkv * sequences >= (own * sequences - shared) * device_cus();
 }
 
 int64_t tile_stride(int head_dim) { return head_dim == 128 ? PP::BUF : PW256::IMG; }

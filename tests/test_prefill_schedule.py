@@ -56,11 +56,11 @@ def test_long_chunks_beside_short_ones(replay, hkv, d, chunks):
 
 @pytest.mark.parametrize("hkv,d,chunk,n,shared", [
     # one launch costs less than images of each chunk's own
-    (2, 256, (150, 2150), 8, 8), (4, 256, (150, 5150), 2, 2), (4, 256, (300, 2300), 8, 8), (2, 256, (1000, 1000), 4, 4),
-    (2, 256, (150, 16384), 4, 4),
+    (2, 256, (150, 2150), 8, 8), (2, 256, (150, 5150), 2, 2), (4, 256, (300, 2300), 8, 8), (2, 256, (1000, 1000), 4, 4),
+    (2, 256, (150, 9000), 4, 4), (4, 128, (1000, 9000), 8, 8),
     (4, 128, (150, 300), 8, 8), (2, 128, (300, 2300), 2, 2), (4, 128, (300, 65536), 1, 1), (4, 128, (2000, 2000), 4, 4),
     # images pay although a launch is shared, or the chunk is alone
-    (2, 256, (150, 16384), 2, 0), (4, 256, (512, 8289), 4, 0), (2, 256, (150, 33000), 2, 0), (4, 256, (300, 2300), 1, 0), (4, 128, (4224, 32768), 2, 0),
+    (2, 256, (150, 9000), 2, 0), (4, 128, (1000, 9000), 2, 0), (4, 256, (512, 8289), 4, 0), (2, 256, (150, 33000), 2, 0), (4, 256, (300, 2300), 1, 0), (4, 128, (4224, 32768), 2, 0),
     (4, 128, (1999, 1999), 1, 0),
 ])
 def test_a_chunk_leaves_the_shared_launch_where_images_pay(replay, hkv, d, chunk, n, shared):
