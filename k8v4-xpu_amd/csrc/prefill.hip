@@ -26,13 +26,16 @@
 //    relative, 1.8e-3 with the factor rounded to fp16 first), in place as a
 //    packed fp16 multiply by the rounded factor.
 //  * Online softmax in the exp2 domain with a lazy rescale (the running max
-//    only moves when a row's max grows by more than 2^2).
+//    only moves when a row's max grows by more than 2^2; in the kernels of
+//    64-row waves 2^8, where P' then stays a finite fp16).
 //  * Head dim 128 (run_segment_pp): eight waves in two groups that alternate
 //    between matrix and vector work half a page apart, so each SIMD's matrix
 //    core and vector ALU run side by side.  V is dequantized into the tile
 //    ((nibble - v_zero) * v_scale / 16, one fp16 rounding) and the softmax
 //    row sums come from the PV product itself (an extra MFMA against a ones
-//    row), so the softmax is max, exp2 and one conversion per score.
+//    row), so the softmax is max, exp2 and one conversion per score.  Over tile
+//    images the row sums stay fp32, and long segments run on four waves of 64
+//    rows (run_segment_wide).
 //  * Head dim 256 over tile images (run_segment_pair): two waves share 64 rows
 //    and interleave the vector work with the products in their own instruction
 //    streams.  In place (run_segment): four waves of 32 rows that convert each
@@ -1790,9 +1793,8 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
 // from LDS for two MFMAs (a 32-row wave: one), the page order keeps the tile
 // reads in L2 (7.0 -> 0.9 GB a head from beyond it), and a running max that may
 // lag by 2^8 rescales the 128 accumulators rarely (a lag of 2^2 cost 8 %).
-// Measured, 4,224 query tokens over 135,296 keys, 4 KV heads, against two
-// groups of four 32-row waves in ping-pong: 6,080 -> 5,790 us (1,137 -> 1,194
-// TFLOP/s).
+// Measured, 4,224 query tokens over 131,072 cached, 4 KV heads, against two groups
+// of four 32-row waves in ping-pong: 6,366 -> 6,156 us (1,086 -> 1,123 TFLOP/s).
 //
 // With no second wave on the SIMD to overlap with, the wave's own instruction
 // stream carries three pages at once, one MFMA per slot with the vector work
@@ -1811,9 +1813,8 @@ __device__ __forceinline__ void run_segment_pair(const PrefillArgs &a, char *sme
 // slot (i + 2) % 4 held V(i - 2), last read in iteration i - 1.
 struct PW128 {
   static constexpr int D = 128;
-  static constexpr int NW = 4, THREADS = 256, ROWS = 256;
+  static constexpr int THREADS = 256, ROWS = 256;
   static constexpr int SLOTS = 4;
-  static constexpr int PIECES = 9;  // per wave and group: 35 pieces, one of them moved twice
   static constexpr int LDS = SLOTS * PP::BUF;
   static_assert(PP::V_OFF == 17 * 1024 && PP::BUF == 35 * 1024, "piece assignment of the DMAs");
   static_assert(ROWS == Tile<128>::ROWS, "one block shape per head dim");
@@ -2139,7 +2140,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(Tile<D>::THREADS, Tile<D>:
                           amdgpu_waves_per_eu(Tile<D>::WPE, Tile<D>::WPE))) void
 prefill_kernel(PrefillArgs a) {
   using T = Tile<D>;
-  static_assert(D == 128 || !PRE, "head dim 256 over tile images: prefill_tiles256_kernel");
+  static_assert(D == 128 || !PRE, "head dim 256 over tile images: prefill_tiles_kernel<256>");
   constexpr int LDS_BYTES = D == 128 ? PP::LDS : 2 * T::BUF + T::STAGE;
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
   const int w = blockIdx.x;
@@ -2173,7 +2174,7 @@ prefill_kernel(PrefillArgs a) {
 }
 
 // Dequantizes every page of a KV head (blockIdx.y) once into its tile image (the
-// LDS layout of run_segment_pp's ring): one work-group of 256 threads per page.
+// LDS layout of the 128-dim rings): one work-group of 256 threads per page.
 // The page's V codes and scale planes are staged in LDS with coalesced loads
 // in the order the in-kernel conversion stages them; then each thread
 // dequantizes two K chunks (read directly) and two V items with the same
@@ -2217,11 +2218,10 @@ __global__ __launch_bounds__(256) void prefill_convert_kernel(PrefillArgs a, cha
   }
 }
 
-// D = 256: every page of a KV head dequantized once into its tile image (the
-// LDS layout run_segment multiplies from), one work-group of four waves per
-// page: the page is staged and converted exactly as the attention kernel
-// does in place, then the image leaves LDS with nontemporal 16-byte stores
-// (TBUF bytes: the tail past BUF carries staged codes nothing reads).
+// D = 256: every page of a KV head (blockIdx.y) dequantized once into its tile
+// image (the layout of PW256), one work-group of four waves per page: the page is
+// staged and converted as the in-place kernel does it, K with one rounding, then
+// leaves LDS in the image's order with nontemporal 16-byte stores.
 __global__ __launch_bounds__(256) void prefill_convert256_kernel(PrefillArgs a, char *tiles) {
   using T = Tile<256>;
   static_assert(T::THREADS == 256 && T::KROW == PW256::KROW, "one page per work-group of four waves");
@@ -2473,9 +2473,12 @@ int rows_per_block(int head_dim) { return head_dim == 128 ? Tile<128>::ROWS : Ti
 // in-kernel conversion costs less than the extra tile traffic).
 constexpr int kPreMinBlocks = 4;
 
-// Head dim 256: the calls that only ever ran over tile images, whose workspace
-// has to hold them (62 ns per page and 59 us of launches per KV head against
-// 9 ns per row block and page, with the kernels these figures were taken on).
+// The calls that only ever run over tile images, whose workspace has to hold
+// those of one head at least: what k8v4_prefill_uses_tiles answers.  Callers size
+// workspaces by it, so the line stays where it was first drawn (head dim 256: by a
+// cost per page, per row block and page and per launch that no kernel here has any
+// more); a call on its other side still runs over images where that is faster now,
+// if there is room (images_pay_off).
 bool tiles_pay_off(int64_t nbh, int64_t npages, int head_dim) {
   if (nbh < kPreMinBlocks) return false;
   return head_dim == 128 || (9 * nbh - 62) * npages > 58600;
@@ -2554,12 +2557,13 @@ int heads_per_launch(int64_t npages, int hkv, int head_dim) {
 }
 
 // Head dim 128: 64-row waves (prefill_tiles_kernel) from this many pages per
-// segment on, where a segment is a row block or a work-group's share of one;
-// below it their longer ramp (half a page more than the ping-pong groups')
-// outweighs what they save.  4 heads, ping-pong against 64-row waves: 12 pages
-// 68.2 / 72.8 us, 32 pages 304.8 / 311.9, 34 pages (whole prompt of 4,224
-// tokens) 246 / 273, 49 pages 149.3 / 144.2, 157 pages 355 / 347, 805 pages
-// 6,080 / 5,790.
+// segment on, where a segment is a row block or a work-group's share of one.  4
+// heads, ping-pong / 64-row waves: 3 pages 40.7 / 38.5 us, 12 pages (whole prompt of
+// 1,999 tokens) 60.9 / 56.7, 33 pages (of 4,224) 147 / 140, 50 pages 132 / 124, 126
+// pages 219 / 208, 805 pages 6,366 / 6,156.  Below the line the ping-pong groups stay
+// for their error: with a running max that lags by no more than 2^2 more of the
+// largest probabilities are exact (700 tokens over 1,000, fp16: 5.66e-4 against
+// 5.84e-4 of 64-row waves; 40 shapes of up to 5,000 keys 0.1-4 % less).
 constexpr int kWideMinPages = 40;
 
 // Host mirror of the device schedule; false if the call is too large for it.

@@ -342,11 +342,11 @@ class Xe2K8V4Impl(AttentionImpl[Xe2K8V4Metadata]):
 
 
 # ----------------------------------------------------------------- helpers
-# Chunks the single prefill entry would run with its in-kernel page conversion
-# gain nothing from running alone: a step's share one batched launch.  A chunk
-# the single entry serves from per-head tile images (each page dequantized
-# once per KV head: at head dim 128 over 128 tokens; at head dim 256 long
-# chunks over long contexts) runs alone.  The library's plan decides.
+# A chunk the single prefill entry always serves from per-head tile images (each
+# page dequantized once per KV head: at head dim 128 over 128 tokens; at head dim
+# 256 long chunks over long contexts) runs alone.  A step's other chunks go into
+# one batched call, which takes out by itself those whose own images cost less
+# than their part of the shared launch.  The library's plan decides both.
 def _runs_alone(width: int, seq_len: int, layout) -> bool:
     _check_covers(seq_len, width)
     return ops().prefill_uses_tiles(seq_len, width, layout.hkv, layout.head_dim)

@@ -412,9 +412,10 @@ class _Ops:
         return n
 
     def prefill_uses_tiles(self, seq_len: int, q_len: int, hkv: int, head_dim: int) -> bool:
-        """Whether :meth:`prefill_paged` serves this shape from per-KV-head tile
-        images (each page dequantized once per head) rather than converting
-        pages in place as :meth:`prefill_paged_batch` does."""
+        """Whether :meth:`prefill_paged` always serves this shape from per-KV-head
+        tile images (each page dequantized once per head), which its workspace
+        then has to hold.  False: it does so only where the workspace has room
+        and that is faster, and may convert pages in place."""
         n = int(self._lib.k8v4_prefill_uses_tiles(int(seq_len), int(q_len), int(hkv), int(head_dim)))
         _require(n >= 0, "bad shape for the prefill plan")
         return n == 1

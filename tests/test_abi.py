@@ -243,6 +243,6 @@ def test_single_prefill_uses_tile_images_where_they_pay(lib, hkv, d, q_len, ctx,
     seq_len = ctx + q_len
     assert lib.k8v4_prefill_uses_tiles(seq_len, q_len, hkv, d) == int(tiles)
     if tiles:  # the workspace holds one tile image per page beside the partial states
-        stride = 35 * 1024 if d == 128 else 68 * 1024
+        stride = 35 * 1024 if d == 128 else 66 * 1024
         assert lib.k8v4_prefill_workspace_bytes(seq_len, q_len, hkv, d) > -(-seq_len // 64) * stride
     assert lib.k8v4_prefill_uses_tiles(seq_len, seq_len + 1, hkv, d) == -1

@@ -173,7 +173,7 @@ def test_prefill_chunk_4224_over_131072_all_rows(gpu_ops):
 @pytest.mark.parametrize("hkv,q_len,seq_len", [(2, 1500, 7000), (4, 1400, 8000)])
 def test_prefill_d256_over_tile_images_all_rows(gpu_ops, hkv, q_len, seq_len):
     """Head dim 256 with enough row blocks and pages for the per-head tile
-    images (the workspace holds them: one 68 KB image per page).  Every row
+    images (the workspace holds them: one 66 KB image per page).  Every row
     against the torch restatement of the reference's prefill, the first and
     last token of every 128-row block against the float64 oracle; max-abs
     2e-3 with a 1e-2 relative allowance."""
@@ -182,7 +182,7 @@ def test_prefill_d256_over_tile_images_all_rows(gpu_ops, hkv, q_len, seq_len):
 
     print("prefill d=256 tiles hkv=%d q=%d seq=%d" % (hkv, q_len, seq_len), flush=True)
     pages = -(-seq_len // PAGE)
-    assert gpu_ops.prefill_workspace_bytes(seq_len, q_len, hkv, 256) > pages * 68 * 1024
+    assert gpu_ops.prefill_workspace_bytes(seq_len, q_len, hkv, 256) > pages * 66 * 1024
     lay = PageLayout(hkv, 256)
     gen = torch.Generator().manual_seed(q_len + seq_len + hkv)
     cache = Cache(pages + 8, lay)
